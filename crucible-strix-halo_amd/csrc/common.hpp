@@ -309,17 +309,8 @@ constexpr int kPolicyL2 = 16;  // sc1
 __device__ __forceinline__ u32x4_t BufLoad128L2(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
   return __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, kPolicyL2);
 }
-// The same store through a buffer resource: the block at byte offset voff + soff (voff may
-// differ per lane group, soff is uniform), the lane's chunk at + (32 (j >> 2) + 8 t) * 2.
-__device__ __forceinline__ void StorePerm32x8Buf(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff,
-                                                 const float v[8], float scale) {
-  const int j = threadIdx.x & 15, t = j & 3;
-  int h[4];
-  Perm32x8Chunk(v, scale, h);
-  __builtin_amdgcn_raw_buffer_store_b128(u32x4_t{(uint32_t)h[0], (uint32_t)h[1], (uint32_t)h[2], (uint32_t)h[3]}, r,
-                                         voff + (uint32_t)(32 * (j >> 2) + 8 * t) * 2, soff, 0);
-}
-// StorePerm32x8Buf with the quad transpose through LDS instead of DPP exchanges: lane
+// StorePerm32x8 through a buffer resource (the block at byte offset voff + soff, the lane's
+// chunk at + (32 (j >> 2) + 8 t) * 2), with the quad transpose through LDS: lane
 // (q, s) = (lane / 4, lane % 4) writes its pair k to dword 16 q + 4 (k ^ f(q)) + s of the
 // wave's 256-dword area (f(q) = (q >> 1) & 3: each of the four writes covers all 32 banks
 // per half wave), then reads its chunk t = s, 16 bytes at 16 q + 4 (t ^ f(q)) (8
@@ -338,7 +329,10 @@ __device__ __forceinline__ void StorePerm32x8LdsBuf(uint32_t* area, __amdgpu_buf
 #pragma unroll
   for (int k = 0; k < 4; ++k) area[16 * q + 4 * (k ^ f) + te] = h[k];
   const u32x4_t c = *reinterpret_cast<const u32x4_t*>(area + 16 * q + 4 * (t ^ f));
-  __builtin_amdgcn_raw_buffer_store_b128(c, r, voff + (uint32_t)(32 * (j >> 2) + 8 * t) * 2, soff, 0);
+  // The whole offset goes in the VGPR (soffset 0): a 16-byte store with a register soffset
+  // whose data registers the next VALU instruction overwrites stored the new values here (the
+  // compiler adds the wait state this needs only where the soffset is not a register).
+  __builtin_amdgcn_raw_buffer_store_b128(c, r, voff + soff + (uint32_t)(32 * (j >> 2) + 8 * t) * 2, 0, 0);
 }
 
 // N consecutive dwords (N = 1..4) from a buffer.
