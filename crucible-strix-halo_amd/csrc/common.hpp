@@ -278,6 +278,30 @@ __device__ __forceinline__ void StoreF8(float* p, const float v[8]) {
   *reinterpret_cast<float4*>(p + 4) = make_float4(v[4], v[5], v[6], v[7]);
 }
 
+// The output transform of 8 summed elements per lane of a 128-block (sv: the lane's svh, sg:
+// WhtLaneSign()), stored at element at of y.  f16 = 0: WHT in fp32, * (norm * svh) (engine
+// LinOutBlock, engine/exl3/exl3.h:69-82).  f16 = 1: y_h rounded to fp16, WHT, * norm -> fp16,
+// * svh -> fp16 (ref/exl3_ref.py:153-156).
+__device__ __forceinline__ void OutputTransformStore(float v[8], const float sv[8], float sg, int f16, void* y, size_t at) {
+  if (f16) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = RoundH(v[i]);
+  }
+  Wht128x8Signed(v);
+  if (f16) {
+    uint32_t h[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      h[k] = __builtin_bit_cast(uint32_t, __floats2half2_rn(RoundH(v[2 * k] * (sg * kHadNorm)) * sv[2 * k],
+                                                            RoundH(v[2 * k + 1] * (sg * kHadNorm)) * sv[2 * k + 1]));
+    *reinterpret_cast<uint4*>(static_cast<__half*>(y) + at) = make_uint4(h[0], h[1], h[2], h[3]);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] *= sg * (kHadNorm * sv[i]);
+    StoreF8(static_cast<float*>(y) + at, v);
+  }
+}
+
 // Raw buffer resource over [base, base + bytes): loads past the end return zero.  Every
 // resource here is wave-uniform; the explicit lane-0 reads keep it in SGPRs even when the
 // compiler cannot prove the base uniform (a base loaded through a selected pointer would
@@ -333,6 +357,35 @@ __device__ __forceinline__ void StorePerm32x8LdsBuf(uint32_t* area, __amdgpu_buf
   // whose data registers the next VALU instruction overwrites stored the new values here (the
   // compiler adds the wait state this needs only where the soffset is not a register).
   __builtin_amdgcn_raw_buffer_store_b128(c, r, voff + soff + (uint32_t)(32 * (j >> 2) + 8 * t) * 2, 0, 0);
+}
+
+// Asynchronous copies from a buffer into LDS (no registers): lane l's N consecutive dwords (N = 1
+// or 4; the 3-dword form does not pack its lanes) at byte offset voff + soff land at lds + 4 N l
+// (offsets past the buffer give zeros).
+// Written as assembly, so that the compiler's own waits neither count these copies nor hold
+// LDS reads back for them: the caller waits with WaitLoadsBarrier before the reads, and drains
+// the copies before the LDS is used for something else.
+typedef __attribute__((address_space(3))) char LdsChar;
+template <int N>
+__device__ __forceinline__ void CopyToLds(u32x4_t rsrc, uint32_t voff, uint32_t soff, uint32_t lds) {
+  static_assert(N == 1 || N == 4, "a copy moves 1 or 4 dwords per lane");
+  if constexpr (N == 1)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
+  else
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
+}
+// Raw buffer words for CopyToLds (as MakeRsrc).
+__device__ __forceinline__ u32x4_t MakeRsrcWords(const void* base, uint32_t bytes) {
+  const uint64_t a = reinterpret_cast<uint64_t>(base);
+  return u32x4_t{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a),
+                 (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32)) & 0xffffu,
+                 (uint32_t)__builtin_amdgcn_readfirstlane((int)bytes), 0x00020000u};
+}
+// Waits until at most N of the wave's vector memory operations are outstanding (they end in
+// order) and its LDS operations are done, then for the workgroup.
+template <int N>
+__device__ __forceinline__ void WaitLoadsBarrier() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
 // N consecutive dwords (N = 1..4) from a buffer.

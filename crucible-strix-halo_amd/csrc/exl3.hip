@@ -1,5 +1,6 @@
 // EXL3 linear op on MI355X: loader repack, bit-exact dequant, and the linear
 // (input transform -> fused decode/MFMA GEMM -> fixed-order split sum + output transform).
+#include <algorithm>
 #include <vector>
 
 #include "internal.hpp"
@@ -114,22 +115,8 @@ __global__ void __launch_bounds__(256) OutputTransformKernel(XfOutTable t) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) v[i] += p[i];
   }
-  if (J.f16) {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = RoundH(v[i]);
-  }
-  Wht128x8Signed(v);
   LoadH8(J.svh + c0, sv);
-  const float sg = WhtLaneSign();
-  if (J.f16) {
-    __half* d = static_cast<__half*>(J.y) + (size_t)r * J.ldy + c0;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) d[i] = __float2half(RoundH(v[i] * (sg * kHadNorm)) * sv[i]);
-  } else {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] *= sg * (kHadNorm * sv[i]);
-    StoreF8(static_cast<float*>(J.y) + (size_t)r * J.ldy + c0, v);
-  }
+  OutputTransformStore(v, sv, WhtLaneSign(), J.f16, J.y, (size_t)r * J.ldy + c0);
 }
 
 // ---- host side ------------------------------------------------------------------------
@@ -242,6 +229,23 @@ bool LaunchGemmMulti(int k2, int cb, int nrb, const GemmMulti& gm, hipStream_t s
   }
 }
 
+bool LaunchGemmRows(int k2, int cb, const RowsMulti& gm, hipStream_t s) {
+  switch (k2) {
+    case 2: return LaunchGemmRowsRate2(cb, gm, s);
+    case 3: return LaunchGemmRowsRate3(cb, gm, s);
+    case 4: return LaunchGemmRowsRate4(cb, gm, s);
+    case 5: return LaunchGemmRowsRate5(cb, gm, s);
+    case 6: return LaunchGemmRowsRate6(cb, gm, s);
+    case 7: return LaunchGemmRowsRate7(cb, gm, s);
+    case 8: return LaunchGemmRowsRate8(cb, gm, s);
+    case 10: return LaunchGemmRowsRate10(cb, gm, s);
+    case 12: return LaunchGemmRowsRate12(cb, gm, s);
+    case 14: return LaunchGemmRowsRate14(cb, gm, s);
+    case 16: return LaunchGemmRowsRate16(cb, gm, s);
+    default: return false;
+  }
+}
+
 bool LaunchGemmTall(int k2, int cb, dim3 grid, const GemmArgs& g, hipStream_t s) {
   switch (k2) {
     case 2: return LaunchGemmTallRate2(cb, grid, g, s);
@@ -259,11 +263,38 @@ bool LaunchGemmTall(int k2, int cb, dim3 grid, const GemmArgs& g, hipStream_t s)
   }
 }
 
+// The many-row GEMM (Exl3GemmRowsKernel) or the few-row path for M rows of one matrix, by their
+// estimated times in us (whole calls at 4 bpw, 65-4,096 rows of 2048 -> 4096, 4096 -> 2048, 2048 -> 512
+// and 2048 -> 12288 measured: within ~15%).
+//   Few rows: ~13.5 + 9.6 ns per row and 1 M weights.
+//   Many rows: ~6 + per step (32 k) 0.21 + 0.05 per row block while at most 256 workgroups run (one
+//   per CU), 0.37 + 0.0625 per round of 512 (two per CU).
+// Measured, few / many rows: 2048 -> 4096 128 rows 21.6 / 22.9, 256 34 / 26, 2,048 182 / 62; 4096 -> 2048 256
+// rows 34 / 40, 512 54 / 44; 2048 -> 512 512 rows 17 / 23, 1,536 31 / 27.
+// nrb: the row blocks per entry of the cheapest many-row form; 0: the few-row path.
+int RowsBlocks(int M, int A, int ncp) {
+  if (M <= 64) return 0;
+  const int blocks = (M + 15) / 16, steps = A / 2;
+  double best = 13.5 + 0.0096e-6 * M * (16.0 * A) * (32.0 * ncp);
+  int nrb = 0;
+  for (int n = 1; n <= std::min(kRowsMaxBlocks, blocks); ++n) {
+    const long wgs = (long)((blocks + n - 1) / n) * (ncp / 4), rem = wgs % 512;
+    const double lone = 0.21 + 0.05 * n, full = 0.37 + 0.0625 * n;
+    const double us = 6.2 + steps * (wgs / 512 * full + (rem == 0 ? 0 : rem <= 256 ? lone : full));
+    if (us < best) {
+      best = us;
+      nrb = n;
+    }
+  }
+  return nrb;
+}
+
 size_t LinearWorkspace(const LinearPlan& p, int I, int O, int M) {
   return AlignUp((size_t)M * I * 2, 256) + AlignUp((size_t)p.S * M * O * 4, 256);
 }
 
-// One group of linears over the same M rows: the grouped input transform, the GEMMs (dense
+// One group of linears over the same M rows: the grouped input transform, then the many-row GEMM
+// with the output transforms in it, or the GEMMs (dense
 // row entries, no device tables; the jobs of one rate and codebook in one launch, up to
 // kMaxMultiJobs a launch), the grouped output transform.  Jobs are checked by the caller;
 // ws holds each job's transformed input and partials.
@@ -305,6 +336,31 @@ int RunGroup(const cx_exl3_job* jobs, int n, int M, char* ws, hipStream_t s) {
     ps[j] = p;
   }
   hipLaunchKernelGGL(InputTransformKernel, dim3((unsigned)((in_items * 16 + 255) / 256)), dim3(256), 0, s, tin);
+  // Many rows: transformed outputs straight from one GEMM, the jobs of one rate and codebook in
+  // one launch.  The group takes it when its largest job does.
+  const int big = (int)(std::max_element(gs.begin(), gs.end(),
+                                         [](const GemmArgs& a, const GemmArgs& b) { return a.A * a.ncp < b.A * b.ncp; }) -
+                        gs.begin());
+  if (RowsBlocks(M, gs[big].A, gs[big].ncp) > 0) {
+    std::vector<bool> done(n, false);
+    for (int j = 0; j < n; ++j) {
+      if (done[j]) continue;
+      RowsMulti gm{};
+      for (int i = j; i < n && gm.n < kMaxMultiJobs; ++i) {
+        if (done[i] || jobs[i].m.k2 != jobs[j].m.k2 || jobs[i].m.codebook != jobs[j].m.codebook) continue;
+        const GemmArgs& g = gs[i];
+        const int nrb = std::max(1, RowsBlocks(M, g.A, g.ncp));
+        const int entries = (M + 16 * nrb - 1) / (16 * nrb);
+        gm.job[gm.n] = RowsJob{g.mat.tiles, g.mat.svh, g.plane[0].x, g.plane[0].y, jobs[i].y, jobs[i].ldy,
+                               jobs[i].y_dtype == CX_F16 ? 1 : 0, M, g.A, g.ncp, ps[i].S, nrb, entries};
+        gm.start[gm.n + 1] = gm.start[gm.n] + RowsJobGroups(entries, g.ncp);
+        ++gm.n;
+        done[i] = true;
+      }
+      if (!LaunchGemmRows(jobs[j].m.k2, jobs[j].m.codebook, gm, s)) return CX_E_UNSUPPORTED;
+    }
+    return LaunchStatus();
+  }
   // Every job has the same row count, so the same row-block count, and the same in-workgroup
   // K split (4): jobs of one rate and codebook can share a launch.
   std::vector<bool> done(n, false);

@@ -1,4 +1,4 @@
-// Exl3GemmPrefillKernel instantiations for one rate (compiled once per rate with
+// Exl3GemmPrefillKernel, Exl3GemmTallKernel and Exl3GemmRowsKernel instantiations for one rate (compiled once per rate with
 // -DCX_RATE=K2).  Built with MFMA accumulators in VGPRs (-amdgpu-mfma-vgpr-form): with
 // accumulator VGPRs the register allocator otherwise copies accumulators between the
 // two register files inside the decode loop.
@@ -60,5 +60,18 @@ bool CX_CAT(LaunchGemmTallRate, CX_RATE)(int cb, dim3 grid, const GemmArgs& g, h
   return false;
 }
 
-}  // namespace cx
+bool CX_CAT(LaunchGemmRowsRate, CX_RATE)(int cb, const RowsMulti& gm, hipStream_t s) {
+  constexpr int K2 = CX_RATE;
+  auto go = [&](auto cbc) {
+    hipLaunchKernelGGL((Exl3GemmRowsKernel<K2, decltype(cbc)::value>), dim3((unsigned)gm.start[gm.n]), dim3(256), 0, s, gm);
+    return true;
+  };
+  if (cb == kCbMul1) return go(IC<kCbMul1>{});
+  if constexpr (K2 % 2 == 0) {
+    if (cb == kCbMcg) return go(IC<kCbMcg>{});
+    if (cb == kCb3Inst) return go(IC<kCb3Inst>{});
+  }
+  return false;
+}
 
+}  // namespace cx

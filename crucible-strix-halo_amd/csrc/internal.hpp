@@ -7,6 +7,7 @@
 
 #include "../../include/crucible_exl3.h"
 #include "gemm.hpp"
+#include "gemm_rows.hpp"
 
 namespace cx {
 
@@ -106,6 +107,8 @@ bool LaunchDecodeStage(int k2, int k2d, int cb, const GemmArgs& gu, const GemmAr
 // Exl3GemmMultiKernel: gm.n jobs (K split over 4 waves) at rate k2, codebook cb, nrb row
 // blocks; gm.start[gm.n] workgroups.
 bool LaunchGemmMulti(int k2, int cb, int nrb, const GemmMulti& gm, hipStream_t s);
+// Exl3GemmRowsKernel: gm.n jobs at rate k2 and codebook cb; gm.start[gm.n] workgroups.
+bool LaunchGemmRows(int k2, int cb, const RowsMulti& gm, hipStream_t s);
 // Per-rate launchers (one translation unit per rate, gemm_inst.hip).
 #define CX_DECLARE_RATE(K2)                                                                          \
   bool LaunchGemmRate##K2(int cb, int nrb, int ksw, dim3 grid, const GemmArgs& g, hipStream_t s); \
@@ -113,7 +116,8 @@ bool LaunchGemmMulti(int k2, int cb, int nrb, const GemmMulti& gm, hipStream_t s
                                  hipStream_t s);                                                         \
   bool LaunchGemmTallRate##K2(int cb, dim3 grid, const GemmArgs& g, hipStream_t s);                         \
   bool LaunchDecodeStageRate##K2(int cb, int k2d, const GemmArgs& gu, const GemmArgs& dn, int nyp, hipStream_t s); \
-  bool LaunchGemmMultiRate##K2(int cb, int nrb, const GemmMulti& gm, hipStream_t s);
+  bool LaunchGemmMultiRate##K2(int cb, int nrb, const GemmMulti& gm, hipStream_t s); \
+  bool LaunchGemmRowsRate##K2(int cb, const RowsMulti& gm, hipStream_t s);
 CX_DECLARE_RATE(2)
 CX_DECLARE_RATE(3)
 CX_DECLARE_RATE(4)
