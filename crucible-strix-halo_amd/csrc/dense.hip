@@ -6,7 +6,8 @@
 //   * more rows, or fp16 x: x rounded to fp16 (the reference packs it first,
 //     PrefillPackKernel) and v_mfma_f32_16x16x32_f16 with fp32 sums: up to 64 rows one
 //     workgroup per 16 outputs with K split over its 8 waves (DenseSplitKernel), above
-//     that tiles of 64 rows x 64 outputs (DenseMfmaKernel).
+//     that tiles of 64 rows x 48-96 outputs through LDS (DenseTileKernel); rows that are not
+//     16-byte aligned, or widths that are no multiple of 64, take DenseMfmaKernel.
 #include "internal.hpp"
 
 namespace cx {
@@ -144,6 +145,120 @@ __global__ void __launch_bounds__(256) DenseMfmaKernel(const __half* __restrict_
     for (int i = 0; i < 4; ++i) {
       const int r = m0 + 4 * (lane >> 4) + i;
       if (r < M) y[(size_t)r * ldy + o] = acc[n][i];
+    }
+  }
+}
+
+// Many rows, 16-byte aligned: a 512-thread workgroup computes rows [64 bx, 64 bx + 64) x outputs
+// [16 NB by, 16 NB (by + 1)).  Chunks of 64 k of its x rows and W rows are copied from memory straight
+// into LDS two chunks ahead, whole 128-byte lines; wave w multiplies row block w / 2 by all NB output
+// blocks over half w % 2 of the chunk's k, and the two halves' sums are added at the end.  Rows >= M
+// and outputs >= O read zeros (buffer bounds) and are not stored.  XF32: x is fp32, rounded to fp16
+// for the product.
+//
+// A router product is small (2,048 x 513 outputs over 2,048 k: 4.3 GFLOP, 23 MB), and the rows and
+// weights that each workgroup reads again (186 MB in all) bound it.  Loading the MFMA fragments
+// from memory (16 bytes from each of 16 rows) gave ~35 bytes per ns and CU: 66 us a call with one
+// wave over all of K (DenseMfmaKernel), 31 us with K split over 8 waves; in whole lines into LDS
+// 15.5 us.  gridDim.x is a multiple of 8, so all workgroups of a row tile run on one XCD and its
+// x rows go into one L2 (3,000 rows: 35 -> 18 us).
+template <bool XF32, int NB>
+__global__ void __launch_bounds__(512) DenseTileKernel(const __half* __restrict__ W, int O, int I,
+                                                       const void* __restrict__ x, int ldx, int M, float* __restrict__ y,
+                                                       int ldy) {
+  constexpr int esz = XF32 ? 4 : 2, XB = 64 * esz;  // bytes of a chunk's x row
+  constexpr int XP = XB / 16;                        // its 16-byte pieces
+  constexpr int XI = 64 * XB / 1024, WI = 2 * NB;    // copies (1 KB each) of a chunk
+  constexpr int NBUF = 3;
+  constexpr int CB = (XI + WI) * 1024;
+  constexpr int NC = (XI + WI) / 8, NX = (XI + WI) % 8;  // copies of every wave; waves with one more
+  __shared__ __align__(16) char smem[NBUF * CB];
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int m0 = blockIdx.x * 64, o0 = blockIdx.y * 16 * NB;
+  if (m0 >= M) return;
+  const int rows = min(64, M - m0), outs = min(16 * NB, O - o0);
+  const u32x4_t rx = MakeRsrcWords(static_cast<const char*>(x) + (size_t)m0 * ldx * esz, (uint32_t)((size_t)rows * ldx * esz));
+  const u32x4_t rw = MakeRsrcWords(W + (size_t)o0 * I, (uint32_t)((size_t)outs * I * 2));
+  // Copy t moves 1024 / XB rows of x (t < XI) or 8 rows of W; lane l the slot l of their pieces.
+  // Piece p of row r lies in slot p ^ (r & 7): the 8 rows of a fragment read cover all banks.
+  const int xr = lane / XP, wr = lane >> 3;
+  const uint32_t lds = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)(LdsChar*)smem);
+  auto copy = [&](int c, int buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i <= NC; ++i) {
+      const int t = 8 * i + wave;
+      if (i == NC && wave >= NX) break;  // wave-uniform
+      const uint32_t dst = lds + buf * CB + t * 1024;
+      if (t < XI) {
+        const int r = t * (1024 / XB) + xr;
+        CopyToLds<4>(rx, (uint32_t)(xr * ldx * esz + 16 * ((lane % XP) ^ (r & 7))),
+                     (uint32_t)(t * (1024 / XB) * ldx * esz + c * XB), dst);
+      } else {
+        CopyToLds<4>(rw, (uint32_t)(wr * I * 2 + 16 * ((lane & 7) ^ wr)), (uint32_t)((t - XI) * 8 * I * 2 + c * 128), dst);
+      }
+    }
+  };
+  const int rb = wave >> 1, kh = wave & 1, ln = lane & 15, q = lane >> 4;
+  const int ar = 16 * rb + ln;
+  // The lane's fragment of its x row (two pieces of fp32, one of fp16) and of W row ln.
+  uint32_t xo[2];
+  xo[0] = (uint32_t)(ar * XB + 16 * ((XF32 ? 8 * kh + 2 * q : 4 * kh + q) ^ (ar & 7)));
+  xo[1] = (uint32_t)(ar * XB + 16 * ((8 * kh + 2 * q + 1) ^ (ar & 7)));
+  const uint32_t wo = (uint32_t)(XI * 1024 + ln * 128 + 16 * ((4 * kh + q) ^ (ln & 7)));
+  float4_t acc[NB];
+#pragma unroll
+  for (int n = 0; n < NB; ++n) acc[n] = float4_t{0.f, 0.f, 0.f, 0.f};
+  const int chunks = I / 64;
+  copy(0, 0);
+  copy(1, 1);
+  int buf = 0;
+  for (int c = 0; c < chunks; ++c) {
+    // Chunk c was asked for two chunks ago: younger than it are one chunk's copies.  After the
+    // barrier every wave's copies are there, and the buffer of the chunk before is free.
+    if (wave < NX)
+      WaitLoadsBarrier<NC + 1>();
+    else
+      WaitLoadsBarrier<NC>();
+    copy(c + 2, buf == 0 ? NBUF - 1 : buf - 1);  // past the last chunk: other columns or zeros, not used
+    const char* sb = smem + buf * CB;
+    half8_t a;
+    if constexpr (XF32) {
+      // Whole-vector casts: element-wise bit casts of ext-vector elements are miscompiled
+      // by this toolchain (every element reads element 0).
+      const float4_t lo = *reinterpret_cast<const float4_t*>(sb + xo[0]);
+      const float4_t hi = *reinterpret_cast<const float4_t*>(sb + xo[1]);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        a[k] = (_Float16)lo[k];
+        a[4 + k] = (_Float16)hi[k];
+      }
+    } else {
+      a = __builtin_bit_cast(half8_t, *reinterpret_cast<const u32x4_t*>(sb + xo[0]));
+    }
+#pragma unroll
+    for (int n = 0; n < NB; ++n) {
+      const half8_t b = __builtin_bit_cast(half8_t, *reinterpret_cast<const u32x4_t*>(sb + wo + 2048 * n));
+      acc[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, acc[n], 0, 0, 0);
+    }
+    buf = buf == NBUF - 1 ? 0 : buf + 1;
+  }
+  WaitLoadsBarrier<0>();  // the last copies: their LDS is used again
+  float4_t* red = reinterpret_cast<float4_t*>(smem) + rb * NB * 64;
+  if (kh) {
+#pragma unroll
+    for (int n = 0; n < NB; ++n) red[n * 64 + lane] = acc[n];
+  }
+  __syncthreads();
+  if (kh) return;
+#pragma unroll
+  for (int n = 0; n < NB; ++n) {
+    const float4_t v = acc[n] + red[n * 64 + lane];
+    const int o = o0 + 16 * n + ln;
+    if (o >= O) continue;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int r = m0 + 16 * rb + 4 * q + i;
+      if (r < M) y[(size_t)r * ldy + o] = v[i];
     }
   }
 }
@@ -300,6 +415,39 @@ int cx_dense_linear(const uint16_t* W, int32_t O, int32_t I, const void* x, int3
         else hipLaunchKernelGGL((DenseSplitKernel<false, 4>), grid, dim3(512), 0, s, w, O, I, x, ldx, M, y, ldy);
         break;
     }
+    return LaunchStatus();
+  }
+  if (I % 64 == 0 && ((size_t)ldx * (x_dtype == CX_F32 ? 4 : 2)) % 16 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
+      reinterpret_cast<uintptr_t>(W) % 16 == 0) {
+    // Outputs per workgroup: 48 to 96, the width whose rounds of 256 workgroups (one per CU) cost
+    // least, a workgroup reading 64 rows and 16 n outputs.  513 outputs are 33 blocks of 16: at 2,048
+    // rows 7 tiles of 80 make 224 workgroups (one round), 9 of 64 make 288.
+    const int mt = (M + 63) / 64, ob = (O + 15) / 16;
+    const int row_cost = x_dtype == CX_F32 ? 8 : 4;
+    int nb = 3;
+    long best = -1;
+    for (int n = 3; n <= 6; ++n) {
+      const long cost = ((long)mt * ((ob + n - 1) / n) + 255) / 256 * (row_cost + n);
+      if (best < 0 || cost <= best) {
+        best = cost;
+        nb = n;
+      }
+    }
+    auto go = [&](auto f32c, auto nbc) {
+      constexpr bool F32 = decltype(f32c)::value != 0;
+      constexpr int NB = decltype(nbc)::value;
+      hipLaunchKernelGGL((DenseTileKernel<F32, NB>), dim3((mt + 7) / 8 * 8, (ob + NB - 1) / NB), dim3(512), 0, s, w, O, I, x, ldx, M, y, ldy);
+    };
+    auto width = [&](auto f32c) {
+      switch (nb) {
+        case 3: go(f32c, IC<3>{}); break;
+        case 4: go(f32c, IC<4>{}); break;
+        case 5: go(f32c, IC<5>{}); break;
+        default: go(f32c, IC<6>{}); break;
+      }
+    };
+    if (x_dtype == CX_F32) width(IC<1>{});
+    else width(IC<0>{});
     return LaunchStatus();
   }
   constexpr int NB = 4;  // 64 outputs per workgroup
