@@ -161,7 +161,7 @@ __global__ void __launch_bounds__(256) DenseMfmaKernel(const __half* __restrict_
 // from memory (16 bytes from each of 16 rows) gave ~35 bytes per ns and CU: 66 us a call with one
 // wave over all of K (DenseMfmaKernel), 31 us with K split over 8 waves; in whole lines into LDS
 // 15.5 us.  gridDim.x is a multiple of 8, so all workgroups of a row tile run on one XCD and its
-// x rows go into one L2 (3,000 rows: 35 -> 18 us).
+// x rows go into one L2 (3,000 rows: 35 -> 20 us).
 template <bool XF32, int NB>
 __global__ void __launch_bounds__(512) DenseTileKernel(const __half* __restrict__ W, int O, int I,
                                                        const void* __restrict__ x, int ldx, int M, float* __restrict__ y,
