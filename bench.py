@@ -43,8 +43,8 @@ def uses_stage(M):
     return os.environ.get("CX_STAGE", "1") != "0" and M * (TOPK + 1) > 128 and M <= 64
 # The prefill GEMM instantiations this build launches: (profile entry, kernel) per stage.
 PREFILL_KERNELS = {
-    "config4": {"gate_up": ("config 4 gate/up + fused mid", "Exl3GemmPrefillKernel<8, 2, 4, 1, 4, true>"),
-                "down": ("config 4 down", "Exl3GemmPrefillKernel<8, 2, 4, 1, 4, false>")},
+    "config4": {"gate_up": ("config 4 gate/up + fused mid", "Exl3GemmPrefillMidKernel<8, 2>"),
+                "down": ("config 4 down", "Exl3GemmPrefillKernel<8, 2, 4, 1, 4>")},
     "config5": {"gate_up": ("config 5 gate/up (3 bpw)", "Exl3GemmTallKernel<6, 2, 3>"),
                 "down": ("config 5 down (5 bpw)", "Exl3GemmTallKernel<10, 2, 3>")},
 }

@@ -124,8 +124,8 @@ struct GemmArgs {
   // (rows at or above xmap_n read row p).  Decode GEMM only.
   const int* xmap;
   int xmap_n;
-  // Gate/up GEMMs with the mid fused in (Exl3GemmPrefillKernel<..., MID = true>, and the
-  // tall GEMM with tall_seq_mid): the down projection's packed input scales [E + 1][O]
+  // Gate/up GEMMs with the mid fused in (Exl3GemmPrefillMidKernel, and the tall GEMM with
+  // tall_seq_mid): the down projection's packed input scales [E + 1][O]
   // and its input rows xd [rows][O] fp16 (MFMA row order), row p at xd + p * O.  The
   // decode down GEMM's prologue mid (MIDX) reads mid_suh too.
   const __half* mid_suh;
@@ -657,15 +657,8 @@ __device__ __forceinline__ GridPos XcdEntryMajor() {
 // tile of a step (16 NRBT rows x 32 inputs) is loaded once into LDS and shared by the
 // waves, so more waves per workgroup read the activations fewer times.  One barrier per
 // step double-buffers the activation tile.
-//
-// MID: gate and up in one workgroup (2 WPG waves: the first WPG on gate, the others on up,
-// each plane with its own activation tiles), and the mid computed in the epilogue from
-// both planes' sums (MidBlock), written as the down projection's input rows; the raw
-// gate / up sums never leave the workgroup.  Needs 32 WPG CPWV = 128 (one block).
-template <int K2, int CB, int NRBT, int CPWV, int WPG, bool MID = false>
-__global__ void __launch_bounds__(64 * WPG * (MID ? 2 : 1)) Exl3GemmPrefillKernel(GemmArgs g) {
-  static_assert(!MID || 32 * WPG * CPWV == 128, "the fused mid needs one 128-column block per workgroup");
-  constexpr int NP = MID ? 2 : 1;       // planes per workgroup
+template <int K2, int CB, int NRBT, int CPWV, int WPG>
+__global__ void __launch_bounds__(64 * WPG) Exl3GemmPrefillKernel(GemmArgs g) {
   constexpr int T = TileDwords(K2);
   constexpr int SD = 4 * T;
   constexpr int DPL = (SD + 63) / 64;
@@ -678,14 +671,14 @@ __global__ void __launch_bounds__(64 * WPG * (MID ? 2 : 1)) Exl3GemmPrefillKerne
   // and 1.13 with rows padded to 48 halves (the launch times did not change).
   constexpr int XS = 32;
   auto xcol = [](int r, int c) { return 8 * (c ^ ((r >> 1) & 3)); };
-  constexpr int NT = 64 * WPG;             // threads per plane
+  constexpr int NT = 64 * WPG;             // threads
   constexpr int XL = (R * 4 + NT - 1) / NT;  // 16-byte activation loads per thread per step
   // The epilogue stages 16-row slabs (8.4 KB), so the activation tiles set the LDS size and
   // more workgroups fit a CU.
   constexpr int ER = 16;
   constexpr int NXB = 4;  // activation tile buffers (written for s + 1, read by the MFMAs of s - 1)
-  constexpr int XBYTES = NP * NXB * R * XS * 2, EBYTES = NP * ER * 132 * 4;
-  __shared__ uint32_t stage[NP * WPG][CPWV][StageDwords<K2, DPL>()];
+  constexpr int XBYTES = NXB * R * XS * 2, EBYTES = ER * 132 * 4;
+  __shared__ uint32_t stage[WPG][CPWV][StageDwords<K2, DPL>()];
   // Activation tiles during the main loop; the epilogue's row staging afterwards.
   __shared__ __align__(16) char smem[XBYTES > EBYTES ? XBYTES : EBYTES];
   const int n_entries = g.n_entries ? *g.n_entries : g.n_entries_host;
@@ -695,10 +688,9 @@ __global__ void __launch_bounds__(64 * WPG * (MID ? 2 : 1)) Exl3GemmPrefillKerne
   const int4 ent = EntryOf(g, ei);
   const int cpg = gp.x;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int plane = MID ? wave / WPG : 0, lw = MID ? wave % WPG : wave;  // plane, wave within it
-  const int tp = (int)threadIdx.x - plane * NT;                            // thread within the plane
-  const GemmPlane& pl = g.plane[MID ? plane : gp.z];
-  __half(*xs)[R][XS] = reinterpret_cast<__half(*)[R][XS]>(smem + plane * (XBYTES / NP));
+  const int tp = (int)threadIdx.x;
+  const GemmPlane& pl = g.plane[gp.z];
+  __half(*xs)[R][XS] = reinterpret_cast<__half(*)[R][XS]>(smem);
   const int steps = g.A / 2;
   const int row0 = ent.y, nrows = ent.z;
   const int nrb = (nrows + 15) / 16;
@@ -708,7 +700,7 @@ __global__ void __launch_bounds__(64 * WPG * (MID ? 2 : 1)) Exl3GemmPrefillKerne
   __amdgpu_buffer_rsrc_t rw[CPWV];
 #pragma unroll
   for (int c = 0; c < CPWV; ++c) {
-    const int cp = (cpg * WPG + lw) * CPWV + c;
+    const int cp = (cpg * WPG + wave) * CPWV + c;
     rw[c] = MakeRsrc(m.tiles + (size_t)cp * g.A * 2 * T, (uint32_t)steps * SD * 4);
   }
   uint32_t woff[2][ND];
@@ -861,42 +853,6 @@ __global__ void __launch_bounds__(64 * WPG * (MID ? 2 : 1)) Exl3GemmPrefillKerne
     (void)((na == Is + 1 ? (main_loop(integral_constant<int, Is + 1>{}), true) : false) || ...);
   }(std::make_integer_sequence<int, NRBT>{});
 
-  if constexpr (MID) {
-    // Mid per 16-row slab: both planes' raw sums staged in LDS, then one row's block per
-    // 16 lanes of the first 16 ER threads.
-    float(*eb)[ER][132] = reinterpret_cast<float(*)[ER][132]>(smem);
-    const MatPtr mg = MatOf(g, g.plane[0], ent.x), mu = MatOf(g, g.plane[1], ent.x);
-    const int j = threadIdx.x & 15, c0 = cpg * 128 + 8 * j;
-    const int O = g.ncp * 32;
-    for (int r0 = 0; r0 < nrows; r0 += ER) {
-#pragma unroll
-      for (int i = 0; i < NRBT; ++i) {
-        if (i * 16 < r0 || i * 16 >= r0 + ER) continue;
-        const int cl = lw * 32 + ((lane & 15) >> 3) * 16 + (lane & 7);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int r = i * 16 - r0 + 4 * (lane >> 4) + e;
-          eb[plane][r][cl] = acc[i][0][0][e];
-          eb[plane][r][cl + 8] = acc[i][0][1][e];
-        }
-      }
-      __syncthreads();
-      const int rr = threadIdx.x >> 4;
-      if (rr < ER && r0 + rr < nrows) {
-        float gv[8], uv[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          gv[e] = eb[0][rr][8 * j + e];
-          uv[e] = eb[1][rr][8 * j + e];
-        }
-        const size_t p = (size_t)(row0 + r0 + rr);
-        MidBlock(gv, uv, mg.svh + c0, mu.svh + c0, g.mid_suh + (size_t)ent.x * O + c0,
-                 g.mid_xd + p * O + cpg * 128);
-      }
-      __syncthreads();
-    }
-    return;
-  }
   if (pl.epi >= 1) {
     // Output transform per 128-column block: stage y_h rows in LDS, ER rows at a time
     // (reusing the activation tile area), WHT128 * norm * svh per row.
@@ -961,6 +917,197 @@ __global__ void __launch_bounds__(64 * WPG * (MID ? 2 : 1)) Exl3GemmPrefillKerne
       }
     }
   }
+}
+
+}  // namespace cx
+
+namespace cx {
+
+// Gate/up GEMM of short prefill entries (up to 64 rows) with the mid in its epilogue: a workgroup = 8
+// waves owns 128 columns of one entry, waves 0-3 of the gate plane, 4-7 of the up plane, each wave
+// one column pair (B fragments in its registers) x all the rows, full K; the raw sums never leave
+// the workgroup.  Each plane's rows go through LDS in chunks of 64 k (whole 128-byte lines), two
+// buffers, one barrier per two steps; four waves per SIMD hide the rest.
+//
+// Bound by the decode's issue (289 cycles of a SIMD per wave-step, two column runs) with the MFMAs
+// beside it, which hide about half of their 17 cycles each.  Against 32-k activation tiles (64-byte
+// pieces of rows, a barrier per step, three waves per SIMD), gate/up with the mid: 2,048 Zipf-routed
+// rows at 4 bpw 271 -> 253 us, 199 rows 189 -> 166, 600 rows 209 -> 183, 2,048 rows at 8 bpw 364 -> 296.
+template <int K2, int CB>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) Exl3GemmPrefillMidKernel(GemmArgs g) {
+  constexpr int NRB = 4, WPP = 4;  // row blocks of an entry, waves (column pairs) per plane
+  constexpr int T = TileDwords(K2);
+  constexpr int SD = 4 * T;
+  constexpr int DPL = (SD + 63) / 64;
+  constexpr int ND = WindowDwords(K2);
+  constexpr int NT = 64 * WPP;            // threads per plane
+  constexpr int CBYTES = 16 * NRB * 128;  // an activation chunk: 16 NRB rows x 64 halves
+  constexpr int ER = 32;                  // epilogue slab rows
+  constexpr int XBYTES = 2 * 2 * CBYTES, EBYTES = 2 * ER * 132 * 4;
+  __shared__ uint32_t stage[2 * WPP][StageDwords<K2, DPL>()];
+  __shared__ __align__(16) char smem[XBYTES > EBYTES ? XBYTES : EBYTES];
+  const int n_entries = g.n_entries ? *g.n_entries : g.n_entries_host;
+  const GridPos gp = XcdEntryMajor();
+  const int ei = gp.y + g.entry_base;
+  if (ei >= n_entries) return;
+  const int4 ent = EntryOf(g, ei);
+  const int row0 = ent.y, nrows = ent.z;
+  if (nrows <= 0) return;
+  const int nrb = (nrows + 15) / 16, steps = g.A / 2;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int plane = wave / WPP, lw = wave % WPP;  // plane, wave within it
+  const int tp = (int)threadIdx.x - plane * NT;   // thread within the plane
+  const GemmPlane& pl = g.plane[plane];
+  const MatPtr m = MatOf(g, pl, ent.x);
+  const LaneRun<K2> lr(lane);
+  const int cp = gp.x * WPP + lw;
+  const __amdgpu_buffer_rsrc_t rw = MakeRsrc(m.tiles + (size_t)cp * g.A * 2 * T, (uint32_t)steps * SD * 4);
+  const __amdgpu_buffer_rsrc_t rx = MakeRsrc(pl.x + (size_t)row0 * pl.ldx, (uint32_t)nrows * pl.ldx * 2);
+  uint32_t woff[2][ND];
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int i = 0; i < ND; ++i) woff[j][i] = (uint32_t)StagePad<K2>((2 * j + lr.tile) * T + (lr.d0 + i) % T);
+  const uint32_t loff = (uint32_t)lane * DPL * 4;
+  uint32_t* slot = stage[wave];
+  char* xs = smem + plane * 2 * CBYTES;
+
+  // always_inline: past the inliner's limit the body would become a called function.
+  auto main_loop = [&](auto nac) __attribute__((always_inline)) {
+    constexpr int NA = decltype(nac)::value;
+    // Chunk c: 16 NA rows x 8 pieces of 16 bytes.  Thread tp moves piece u = tp % 8 of rows
+    // tp / 8 + 32 i.  In LDS, fragment order: row block, step j = u / 4, k-group u % 4, row ^ u: the 8
+    // pieces of a row, and the 8 rows of a fragment read, each lie in distinct banks.
+    constexpr int XL = (NA + 1) / 2;
+    const int u = tp & 7;
+    uint32_t xoff[XL], xst[XL];
+#pragma unroll
+    for (int i = 0; i < XL; ++i) {
+      const int row = tp / 8 + 32 * i;
+      xoff[i] = (uint32_t)(row * pl.ldx * 2 + 16 * u);
+      xst[i] = (uint32_t)((row >> 4) * 2048 + ((u >> 2) * 64 + (u & 3) * 16 + ((row & 15) ^ u)) * 16);
+    }
+    auto load_x = [&](u32x4_t (&xv)[XL], int c) {
+#pragma unroll
+      for (int i = 0; i < XL; ++i) xv[i] = BufLoad128(rx, xoff[i], (uint32_t)c * 128);
+    };
+    auto store_x = [&](const u32x4_t (&xv)[XL], int buf) {
+#pragma unroll
+      for (int i = 0; i < XL; ++i)
+        if (32 * (i + 1) <= 16 * NA || tp < 128) *reinterpret_cast<u32x4_t*>(xs + buf * CBYTES + xst[i]) = xv[i];
+    };
+    uint32_t xrd[2];  // the lane's fragment of the chunk's step j, row block 0
+#pragma unroll
+    for (int j = 0; j < 2; ++j) xrd[j] = (uint32_t)((64 * j + (lane & 48) + ((lane & 15) ^ (4 * j + (lane >> 4)))) * 16);
+    auto read_windows = [&](uint32_t (&v)[2][3]) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+#pragma unroll
+        for (int i = 0; i < ND; ++i) v[j][i] = slot[woff[j][i]];
+        if constexpr (ND == 2) v[j][2] = 0u;
+      }
+    };
+    auto decode = [&](const uint32_t (&v)[2][3], half8_t (&b)[2]) __attribute__((always_inline)) {
+      half4_t lo0, hi0, lo1, hi1;
+      DecodeRun<K2, CB>(v[0][0], v[0][1], v[0][2], lr.shift, lo0, hi0);
+      DecodeRun<K2, CB>(v[1][0], v[1][1], v[1][2], lr.shift, lo1, hi1);
+      b[0] = half8_t{lo0[0], lo0[1], lo0[2], lo0[3], lo1[0], lo1[1], lo1[2], lo1[3]};
+      b[1] = half8_t{hi0[0], hi0[1], hi0[2], hi0[3], hi1[0], hi1[1], hi1[2], hi1[3]};
+    };
+    constexpr int PFW = 4;  // weight steps in flight
+    Dwords<DPL> wq[PFW];
+    u32x4_t xq[XL];
+    float4_t acc[NA][2];
+#pragma unroll
+    for (int i = 0; i < NA; ++i) acc[i][0] = acc[i][1] = float4_t{0.f, 0.f, 0.f, 0.f};
+    // Loads are unconditional, also past the last step (outside the buffer resources, or other
+    // columns of the rows), so the compiler can count the loads in flight.
+#pragma unroll
+    for (int k = 0; k < PFW; ++k) wq[k] = BufLoadN<DPL>(rw, loff, (uint32_t)k * SD * 4);
+    load_x(xq, 0);
+    half8_t b[2];
+    {
+      // Step 0 decoded, step 1 staged, chunk 0 in LDS, chunk 1 on its way.
+      StageWrite<K2, DPL>(slot, lane, wq[0].v);
+      wq[0] = BufLoadN<DPL>(rw, loff, (uint32_t)PFW * SD * 4);
+      __builtin_amdgcn_wave_barrier();
+      uint32_t v[2][3];
+      read_windows(v);
+      __builtin_amdgcn_wave_barrier();
+      StageWrite<K2, DPL>(slot, lane, wq[1].v);
+      wq[1] = BufLoadN<DPL>(rw, loff, (uint32_t)(PFW + 1) * SD * 4);
+      store_x(xq, 0);
+      load_x(xq, 1);
+      decode(v, b);
+    }
+    for (int s0 = 0; s0 < steps; s0 += 4) {  // steps is a multiple of 4
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int s = s0 + q, buf = q >> 1, j = q & 1;
+        if (j == 0) {
+          __syncthreads();  // chunk s / 2 is written, the other buffer's reads are done
+          store_x(xq, buf ^ 1);
+          load_x(xq, (s >> 1) + 2);
+        }
+        // Windows of step s + 1, then step s + 2 into the slot (the wave's LDS operations run in order).
+        __builtin_amdgcn_wave_barrier();
+        uint32_t v[2][3];
+        read_windows(v);
+        __builtin_amdgcn_wave_barrier();
+        StageWrite<K2, DPL>(slot, lane, wq[(q + 2) % PFW].v);
+        wq[(q + 2) % PFW] = BufLoadN<DPL>(rw, loff, (uint32_t)(s + 2 + PFW) * SD * 4);
+        __builtin_amdgcn_wave_barrier();
+        half8_t av[NA];
+#pragma unroll
+        for (int i = 0; i < NA; ++i)
+          av[i] = __builtin_bit_cast(half8_t, *reinterpret_cast<const u32x4_t*>(xs + buf * CBYTES + i * 2048 + xrd[j]));
+        half8_t nb[2];
+        decode(v, nb);
+#pragma unroll
+        for (int i = 0; i < NA; ++i) {
+          acc[i][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[i], b[0], acc[i][0], 0, 0, 0);
+          acc[i][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[i], b[1], acc[i][1], 0, 0, 0);
+        }
+        b[0] = nb[0];
+        b[1] = nb[1];
+      }
+    }
+    __syncthreads();  // the slabs reuse the activation chunks
+    // The mid per 32-row slab: both planes' raw sums staged in LDS, one row's block per 16 lanes.
+    float(*eb)[ER][132] = reinterpret_cast<float(*)[ER][132]>(smem);
+    const int cl = lw * 32 + ((lane & 15) >> 3) * 16 + (lane & 7), O = g.ncp * 32;
+    const MatPtr mg = MatOf(g, g.plane[0], ent.x), mu = MatOf(g, g.plane[1], ent.x);
+    const int j = threadIdx.x & 15, rr = threadIdx.x >> 4, c0 = gp.x * 128 + 8 * j;
+    for (int i0 = 0; i0 < NA; i0 += 2) {
+#pragma unroll
+      for (int i = 0; i < NA; ++i) {
+        if (i < i0 || i >= i0 + 2) continue;  // uniform
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          float* r = eb[plane][16 * (i & 1) + 4 * (lane >> 4) + k];
+          r[cl] = acc[i][0][k];
+          r[cl + 8] = acc[i][1][k];
+        }
+      }
+      __syncthreads();
+      const int r = 16 * i0 + rr;
+      if (r < nrows) {  // uniform over the row's 16 lanes
+        const size_t p = (size_t)(row0 + r);
+        float gv[8], uv[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          gv[k] = eb[0][rr][8 * j + k];
+          uv[k] = eb[1][rr][8 * j + k];
+        }
+        MidBlock(gv, uv, mg.svh + c0, mu.svh + c0, g.mid_suh + (size_t)ent.x * O + c0, g.mid_xd + p * O + gp.x * 128);
+      }
+      __syncthreads();
+    }
+  };
+  using std::integral_constant;
+  [&]<int... Is>(std::integer_sequence<int, Is...>) __attribute__((always_inline)) {
+    (void)((nrb <= Is + 1 ? (main_loop(integral_constant<int, Is + 1>{}), true) : false) || ...);
+  }(std::make_integer_sequence<int, NRB>{});
 }
 
 }  // namespace cx

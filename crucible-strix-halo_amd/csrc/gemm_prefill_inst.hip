@@ -1,4 +1,4 @@
-// Exl3GemmPrefillKernel, Exl3GemmTallKernel and Exl3GemmRowsKernel instantiations for one rate (compiled once per rate with
+// Instantiations of the prefill and many-row GEMM kernels for one rate (compiled once per rate with
 // -DCX_RATE=K2).  Built with MFMA accumulators in VGPRs (-amdgpu-mfma-vgpr-form): with
 // accumulator VGPRs the register allocator otherwise copies accumulators between the
 // two register files inside the decode loop.
@@ -24,7 +24,7 @@ bool CX_CAT(LaunchGemmPrefillRate, CX_RATE)(int cb, int nrbt, int wpg, bool mid,
   auto shape = [&](auto cbc) {
     if (mid) {  // gate and up in one workgroup, the mid in the epilogue
       if (nrbt != 4 || wpg != 4) return false;
-      hipLaunchKernelGGL((Exl3GemmPrefillKernel<K2, decltype(cbc)::value, 4, 1, 4, true>), grid, dim3(512), 0, s, g);
+      hipLaunchKernelGGL((Exl3GemmPrefillMidKernel<K2, decltype(cbc)::value>), grid, dim3(512), 0, s, g);
       return true;
     }
     if (nrbt == 4 && wpg == 4) return go(cbc, IC<4>{}, IC<4>{});
