@@ -203,13 +203,21 @@ __device__ int BlockExclusiveScan(int v, int* scratch, int* total) {
   return before;
 }
 
-// Stable append of one route per thread (route index i in thread order; e < 0: none):
-// its position is cursor[e] + (routes of expert e in earlier waves) + (earlier lanes of
-// this wave with expert e).  Lanes of one expert are found by ballots over the id bits;
-// the waves take their cursor ranges in wave order, so positions follow route order.
-// Returns the position (or -1).  All threads of the block must call it.
-// nw: waves that may hold valid routes (the others have e < 0); uniform over the block.
-__device__ int StableAppend(int e, int* cursor, int nw) {
+// Stable positions without one wave waiting for another: a workgroup's waves hold consecutive
+// segments of the routes, and each wave counts its own routes per expert in its own counters
+// (LDS, wave w: cnt[w]).  A route's position is the expert's offset + the counts of earlier waves
+// (WavePrefix) + its place among its own wave's routes (WaveAppend).
+using WaveCounts = uint16_t[16][kMaxExperts];
+
+// Zeroes the wave's own counters.
+__device__ void WaveClear(WaveCounts& cnt, int E) {
+  for (int i = threadIdx.x & 63; i < E; i += 64) cnt[threadIdx.x >> 6][i] = 0;
+  __builtin_amdgcn_wave_barrier();  // the wave's LDS operations run in order
+}
+
+// Counts one route per lane (expert e; e < 0: none, in lane order) and returns its place among the
+// wave's routes of that expert so far.  Lanes of one expert are found by ballots over the id bits.
+__device__ int WaveAppend(int e, WaveCounts& cnt) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const bool valid = e >= 0;
   unsigned long long peers = __ballot(valid);
@@ -222,12 +230,25 @@ __device__ int StableAppend(int e, int* cursor, int nw) {
   const int rank = __popcll(peers & ((1ull << lane) - 1ull));
   const int leader = valid ? __ffsll((long long)peers) - 1 : lane;
   int base = 0;
-  for (int ww = 0; ww < nw; ++ww) {
-    if (w == ww && valid && rank == 0) base = atomicAdd(&cursor[e], __popcll(peers));
-    __syncthreads();
+  if (valid && rank == 0) {
+    base = cnt[w][e];
+    cnt[w][e] = (uint16_t)(base + __popcll(peers));
   }
-  base = __shfl(base, leader, 64);
-  return valid ? base + rank : -1;
+  __builtin_amdgcn_wave_barrier();
+  return __shfl(base, leader, 64) + rank;
+}
+
+// Expert e's counts of waves [0, nw) -> their exclusive prefix; returns the sum.
+__device__ int WavePrefix(int e, int nw, WaveCounts& cnt) {
+  int sum = 0;
+#pragma unroll
+  for (int w = 0; w < 16; ++w) {
+    if (w >= nw) break;  // uniform
+    const int c = cnt[w][e];
+    cnt[w][e] = (uint16_t)sum;
+    sum += c;
+  }
+  return sum;
 }
 
 // An expert id in [0, E), or -1 for an id outside it (such a route is dropped).
@@ -240,20 +261,28 @@ __device__ void WritePair(const GroupOut& o, int p, int i, int e) {
   if (o.expert) o.expert[p] = e;
 }
 
-// Whole grouping in one 1024-thread workgroup (up to kSmallRoutes routes); sel may be
-// in global memory or in LDS.  ref/prefill_ref.py:37-45.
-__device__ void GroupSmallBody(const int* sel, const GroupOut& o, int* s_cur, int* s_scan) {
-  const int n = o.M * o.topk;
+// Whole grouping in one 1024-thread workgroup (up to kSmallRoutes = 2 x 1024 routes); sel may be
+// in global memory or in LDS.  ref/prefill_ref.py:37-45.  Latency-bound, one workgroup on one CU: three
+// barriers of the scan and two more, whatever the number of waves.  With the waves taking turns
+// at shared cursors (a barrier per wave and 1,024 routes) 1,990 routes took 9.7 us, now 8.0.
+__device__ void GroupSmallBody(const int* sel, const GroupOut& o, int* s_cur, int* s_scan, WaveCounts& s_cnt) {
+  const int n = o.M * o.topk, per = n > 1024 ? 2 : 1;  // routes per thread
+  const int i0 = ((int)threadIdx.x >> 6) * 64 * per + ((int)threadIdx.x & 63), nw = (n + 64 * per - 1) / (64 * per);
+  int re[2], rl[2];
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {  // ids outside [0, E) are dropped
+    const int i = i0 + 64 * k;
+    re[k] = k < per && i < n ? ValidExpert(sel[i], o.E) : -1;
+  }
   for (int i = threadIdx.x; i < o.nzero; i += blockDim.x) o.zero[i * kStageCtrStride] = 0;
-  for (int e = threadIdx.x; e < o.E; e += blockDim.x) s_cur[e] = 0;
-  __syncthreads();
-  for (int i = threadIdx.x; i < n; i += blockDim.x) {  // counts only; ids outside [0, E) are dropped
-    const int e = sel[i];
-    if ((unsigned)e < (unsigned)o.E) atomicAdd(&s_cur[e], 1);
+  if ((int)threadIdx.x < 64 * nw) {  // whole waves
+    WaveClear(s_cnt, o.E);
+    rl[0] = WaveAppend(re[0], s_cnt);
+    if (per > 1) rl[1] = WaveAppend(re[1], s_cnt);
   }
   __syncthreads();
   const int e = threadIdx.x;
-  const int cnt = e < o.E ? s_cur[e] : 0;
+  const int cnt = e < o.E ? WavePrefix(e, nw, s_cnt) : 0;
   const int nch = o.entries ? (cnt + o.chunk - 1) / o.chunk : 0;
   // Route and chunk counts scanned together (both < 2^16 here).
   int packed = 0;
@@ -273,18 +302,16 @@ __device__ void GroupSmallBody(const int* sel, const GroupOut& o, int* s_cur, in
     FillEmptyEntries(o, (o.M + o.chunk - 1) / o.chunk + ctotal);
   }
   __syncthreads();
-  for (int base = 0; base < n; base += blockDim.x) {
-    const int i = base + threadIdx.x;
-    const int e = i < n ? ValidExpert(sel[i], o.E) : -1;
-    const int p = StableAppend(e, s_cur, min((int)blockDim.x, n - base + 63) >> 6);
-    if (p >= 0) WritePair(o, p, i, e);
-  }
+#pragma unroll
+  for (int k = 0; k < 2; ++k)
+    if (re[k] >= 0) WritePair(o, s_cur[re[k]] + s_cnt[threadIdx.x >> 6][re[k]] + rl[k], i0 + 64 * k, re[k]);
 }
 
 __global__ void __launch_bounds__(1024) GroupSmallKernel(const int* __restrict__ sel, GroupOut o) {
   __shared__ int s_cur[kMaxExperts];
   __shared__ int s_scan[128];
-  GroupSmallBody(sel, o, s_cur, s_scan);
+  __shared__ WaveCounts s_cnt;
+  GroupSmallBody(sel, o, s_cur, s_scan, s_cnt);
 }
 
 // The gate and up input transforms of one lane's 8 elements of a 128-block (signed
@@ -320,8 +347,9 @@ __global__ void __launch_bounds__(1024) GroupInputKernel(const int* __restrict__
   __shared__ int s_e[kMaxTopK + 1];
   __shared__ int s_cur[kMaxExperts];
   __shared__ int s_scan[128];
+  __shared__ WaveCounts s_cnt;
   if (blockIdx.x == 0) {
-    GroupSmallBody(sel, o, s_cur, s_scan);
+    GroupSmallBody(sel, o, s_cur, s_scan, s_cnt);
     return;
   }
   const int topk = o.topk, M = o.M, nb = H / 128, j = threadIdx.x & 15;
@@ -360,6 +388,7 @@ __global__ void __launch_bounds__(1024) RouteGroupInputKernel(const float* __res
   __shared__ int s_sel[kSmallRoutes];
   __shared__ int s_cur[kMaxExperts];
   __shared__ int s_scan[128];
+  __shared__ WaveCounts s_cnt;
   const int topk = o.topk, M = o.M, E = o.E;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   if (blockIdx.x == 0) {
@@ -369,7 +398,7 @@ __global__ void __launch_bounds__(1024) RouteGroupInputKernel(const float* __res
                       wts + (size_t)r * (topk + 1), s_sel + r * topk);
     }
     __syncthreads();
-    GroupSmallBody(s_sel, o, s_cur, s_scan);
+    GroupSmallBody(s_sel, o, s_cur, s_scan, s_cnt);
     return;
   }
   const int nb = H / 128, j = threadIdx.x & 15;
@@ -414,7 +443,7 @@ __global__ void __launch_bounds__(1024) GroupCountKernel(const int* __restrict__
     if (e >= 0) atomicAdd(&h[e], 1);
   }
   __syncthreads();
-  for (int e = threadIdx.x; e < E; e += blockDim.x) tile_counts[(size_t)e * ntiles + blockIdx.x] = h[e];
+  for (int e = threadIdx.x; e < E; e += blockDim.x) tile_counts[(size_t)blockIdx.x * E + e] = h[e];
 }
 
 // Scan and scatter in one launch, one workgroup per tile: every workgroup reads all tile
@@ -427,16 +456,25 @@ __global__ void __launch_bounds__(1024) GroupScatterKernel(const int* __restrict
                                                            GroupOut o) {
   __shared__ int s_scan[128];
   __shared__ int s_cur[kMaxExperts];
+  __shared__ WaveCounts s_cnt;
   const int e = threadIdx.x, tile = blockIdx.x;
+  // The tile's own routes first: they need no other tile's counts.
+  const int n = o.M * o.topk, i = tile * kTile + threadIdx.x;
+  const int re = i < n ? ValidExpert(sel[i], o.E) : -1;
+  int rl = 0;
+  if (tile < ntiles) {
+    WaveClear(s_cnt, o.E);
+    rl = WaveAppend(re, s_cnt);
+  }
   int cnt = 0, before = 0;
   if (e < o.E) {
     // Independent loads issued 8 at a time (a dependent chain would wait ntiles times).
-    const int* tc = tile_counts + (size_t)e * ntiles;
+    const int* tc = tile_counts + e;
     int t = 0;
     for (; t + 8 <= ntiles; t += 8) {
       int v[8];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) v[i] = tc[t + i];
+      for (int i = 0; i < 8; ++i) v[i] = tc[(size_t)(t + i) * o.E];
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         before += t + i < tile ? v[i] : 0;
@@ -444,7 +482,7 @@ __global__ void __launch_bounds__(1024) GroupScatterKernel(const int* __restrict
       }
     }
     for (; t < ntiles; ++t) {
-      const int v = tc[t];
+      const int v = tc[(size_t)t * o.E];
       before += t < tile ? v : 0;
       cnt += v;
     }
@@ -469,12 +507,9 @@ __global__ void __launch_bounds__(1024) GroupScatterKernel(const int* __restrict
     }
     return;
   }
+  if (e < o.E) WavePrefix(e, 16, s_cnt);  // every wave's counts are written: the scan's barriers lie between
   __syncthreads();
-  const int n = o.M * o.topk;
-  const int i = tile * kTile + threadIdx.x;
-  const int se = i < n ? ValidExpert(sel[i], o.E) : -1;
-  const int p = StableAppend(se, s_cur, min((int)blockDim.x, n - tile * kTile + 63) >> 6);
-  if (p >= 0) WritePair(o, p, i, se);
+  if (re >= 0) WritePair(o, s_cur[re] + s_cnt[threadIdx.x >> 6][re] + rl, i, re);
 }
 
 // ---- activation transforms of the experts ----------------------------------------------
