@@ -20,16 +20,19 @@ namespace cx {
 template <class V>
 __global__ void __launch_bounds__(256) RepackKernel(const V* __restrict__ src, V* __restrict__ dst, int A, int ncp,
                                                     uint32_t U) {
-  const uint32_t row = (uint32_t)ncp * U, u = blockIdx.x * 256 + threadIdx.x;  // units of one a, this thread's
-  if (u >= row) return;
-  const uint32_t cp = u / U, w = u - cp * U;
-  for (int a0 = blockIdx.y * 4; a0 < A; a0 += gridDim.y * 4) {  // A is a multiple of 8
-    V v[4];
+  // Units of one a: up to 2^31 of 16 bytes, 2^33 dwords.
+  using Index = std::conditional_t<sizeof(V) == 16, uint32_t, size_t>;
+  const Index row = (Index)ncp * U;
+  for (Index u = (Index)blockIdx.x * 256 + threadIdx.x; u < row; u += (Index)gridDim.x * 256) {
+    const Index cp = u / U, w = u - cp * U;
+    for (int a0 = blockIdx.y * 4; a0 < A; a0 += gridDim.y * 4) {  // A is a multiple of 8
+      V v[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = src[(size_t)(a0 + i) * row + u];
-    V* d = dst + ((size_t)cp * A + a0) * U + w;
+      for (int i = 0; i < 4; ++i) v[i] = src[(size_t)(a0 + i) * row + u];
+      V* d = dst + ((size_t)cp * A + a0) * U + w;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) d[(size_t)i * U] = v[i];
+      for (int i = 0; i < 4; ++i) d[(size_t)i * U] = v[i];
+    }
   }
 }
 
@@ -439,7 +442,7 @@ int cx_exl3_repack(const int16_t* trellis, int32_t in_features, int32_t out_feat
   auto go = [&](auto unit) {
     using V = decltype(unit);
     const int ncp = B / 2, U = 2 * T * 4 / (int)sizeof(V);
-    const dim3 grid((unsigned)(((size_t)ncp * U + 255) / 256), (unsigned)std::min(A / 4, 65535));
+    const dim3 grid((unsigned)std::min<size_t>(((size_t)ncp * U + 255) / 256, 1 << 16), (unsigned)std::min(A / 4, 65535));
     hipLaunchKernelGGL((RepackKernel<V>), grid, dim3(256), 0, (hipStream_t)stream, reinterpret_cast<const V*>(trellis),
                        reinterpret_cast<V*>(tiles), A, ncp, (uint32_t)U);
   };
