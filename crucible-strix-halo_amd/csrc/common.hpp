@@ -302,6 +302,14 @@ __device__ __forceinline__ void OutputTransformStore(float v[8], const float sv[
   }
 }
 
+// Bytes of `rows` rows of I elements, ld elements apart, from the first row's start to the last row's
+// end: the resource over a caller's rows.  Not rows * ld: where the rows are columns of a wider
+// matrix, that would reach ld - I elements past the last row, possibly past the allocation, and
+// prefetches past the last column would read there.
+__host__ __device__ constexpr uint32_t RowsBytes(int rows, int ld, int I, int esz) {
+  return rows > 0 ? (uint32_t)(((size_t)(rows - 1) * ld + I) * esz) : 0u;
+}
+
 // Raw buffer resource over [base, base + bytes): loads past the end return zero.  Every
 // resource here is wave-uniform; the explicit lane-0 reads keep it in SGPRs even when the
 // compiler cannot prove the base uniform (a base loaded through a selected pointer would

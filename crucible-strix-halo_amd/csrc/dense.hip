@@ -70,7 +70,7 @@ __global__ void __launch_bounds__(256) DenseMfmaKernel(const __half* __restrict_
   const int esz = XF32 ? 4 : 2;
   const int rows = max(0, min(16, M - m0));
   const __amdgpu_buffer_rsrc_t rx =
-      MakeRsrc(static_cast<const char*>(x) + (size_t)m0 * ldx * esz, (uint32_t)((size_t)rows * ldx * esz));
+      MakeRsrc(static_cast<const char*>(x) + (size_t)m0 * ldx * esz, RowsBytes(rows, ldx, I, esz));
   const int outs = max(0, min(16 * NB, O - o0));
   const __amdgpu_buffer_rsrc_t rw = MakeRsrc(W + (size_t)o0 * I, (uint32_t)((size_t)outs * I * 2));
   const uint32_t xoff = (uint32_t)((ln * ldx + kq) * esz);
@@ -177,7 +177,7 @@ __global__ void __launch_bounds__(512) DenseTileKernel(const __half* __restrict_
   const int m0 = blockIdx.x * 64, o0 = blockIdx.y * 16 * NB;
   if (m0 >= M) return;
   const int rows = min(64, M - m0), outs = min(16 * NB, O - o0);
-  const u32x4_t rx = MakeRsrcWords(static_cast<const char*>(x) + (size_t)m0 * ldx * esz, (uint32_t)((size_t)rows * ldx * esz));
+  const u32x4_t rx = MakeRsrcWords(static_cast<const char*>(x) + (size_t)m0 * ldx * esz, RowsBytes(rows, ldx, I, esz));
   const u32x4_t rw = MakeRsrcWords(W + (size_t)o0 * I, (uint32_t)((size_t)outs * I * 2));
   // Copy t moves 1024 / XB rows of x (t < XI) or 8 rows of W; lane l the slot l of their pieces.
   // Piece p of row r lies in slot p ^ (r & 7): the 8 rows of a fragment read cover all banks.
@@ -281,7 +281,7 @@ __global__ void __launch_bounds__(512) DenseSplitKernel(const __half* __restrict
   const int esz = XF32 ? 4 : 2;
   const int outs = max(0, min(16, O - o0));
   const __amdgpu_buffer_rsrc_t rw = MakeRsrc(W + (size_t)o0 * I, (uint32_t)((size_t)outs * I * 2));
-  const __amdgpu_buffer_rsrc_t rx = MakeRsrc(x, (uint32_t)((size_t)M * ldx * esz));
+  const __amdgpu_buffer_rsrc_t rx = MakeRsrc(x, RowsBytes(M, ldx, I, esz));
   const uint32_t woff = (uint32_t)((ln * I + k0 + kq) * 2);
   uint32_t xoff[NRB];
 #pragma unroll

@@ -29,3 +29,28 @@ def test_dense_tiles(M, I, Ot, pad, dt):
     # fp32 sums of exact products: at most I roundings of 2^-24 relative to the sum of magnitudes.
     assert torch.all((yb[:, :Ot].double() - ref).abs() <= I * 2.0**-24 * bound + 1e-30)
     assert torch.all(yb[:, Ot:] == 7.0)
+
+
+# x as columns [off, off + I) of a wider matrix, up to its last column: the storage ends where x does,
+# and NaN stands in every other column.  DenseTileKernel, DenseSplitKernel (up to 64 rows, I a multiple of
+# 256), DenseMfmaKernel (the others), DenseGemvKernel (fp32, up to 8 rows).
+@pytest.mark.parametrize("M,I,Ot,off", [
+    (8192, 2048, 70, 128), (65, 64, 33, 8), (130, 192, 513, 64), (64, 2048, 33, 64), (17, 256, 49, 8), (9, 512, 17, 4),
+    (70, 96, 33, 32), (300, 160, 65, 8), (33, 64, 20, 1), (5, 256, 40, 4),
+])
+@pytest.mark.parametrize("dt", ["float32", "float16"])
+def test_dense_offset_view(M, I, Ot, off, dt):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from exl3moe import ops
+    g = torch.Generator(device="cuda")
+    g.manual_seed(M + I + off)
+    W = torch.randn(Ot, I, device="cuda", generator=g).half()
+    xb = torch.full((M, off + I), float("nan"), device="cuda", dtype=getattr(torch, dt))
+    xb[:, off:] = torch.randn(M, I, device="cuda", generator=g).to(xb.dtype)
+    x = xb[:, off:]
+    y = ops.dense_linear(W, x)
+    xs = (x if dt == "float32" and M <= 8 else x.half()).double()  # up to 8 fp32 rows: fp32 products
+    ref, bound = xs @ W.double().t(), xs.abs() @ W.double().abs().t()
+    # fp32 sums: at most I roundings of the products and I of the sums, 2^-24 each.
+    assert torch.all((y.double() - ref).abs() <= 2 * I * 2.0**-24 * bound + 1e-30)
