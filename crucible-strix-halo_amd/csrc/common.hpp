@@ -373,14 +373,17 @@ __device__ __forceinline__ void StorePerm32x8LdsBuf(uint32_t* area, __amdgpu_buf
 // Written as assembly, so that the compiler's own waits neither count these copies nor hold
 // LDS reads back for them: the caller waits with WaitLoadsBarrier before the reads, and drains
 // the copies before the LDS is used for something else.
+// The compiler puts no wait states into assembly: s_mov and s_nop 3 are the five that lie between a
+// VALU write of a scalar operand (v_readfirstlane, a spilled SGPR's v_readlane) and the load reading
+// it, and the one between the write of m0 and its use.
 typedef __attribute__((address_space(3))) char LdsChar;
 template <int N>
 __device__ __forceinline__ void CopyToLds(u32x4_t rsrc, uint32_t voff, uint32_t soff, uint32_t lds) {
   static_assert(N == 1 || N == 4, "a copy moves 1 or 4 dwords per lane");
   if constexpr (N == 1)
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "memory", "m0");
   else
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "memory", "m0");
 }
 // Raw buffer words for CopyToLds (as MakeRsrc).
 __device__ __forceinline__ u32x4_t MakeRsrcWords(const void* base, uint32_t bytes) {
