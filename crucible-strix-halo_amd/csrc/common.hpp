@@ -294,7 +294,9 @@ __device__ __forceinline__ void OutputTransformStore(float v[8], const float sv[
     for (int k = 0; k < 4; ++k)
       h[k] = __builtin_bit_cast(uint32_t, __floats2half2_rn(RoundH(v[2 * k] * (sg * kHadNorm)) * sv[2 * k],
                                                             RoundH(v[2 * k + 1] * (sg * kHadNorm)) * sv[2 * k + 1]));
-    *reinterpret_cast<uint4*>(static_cast<__half*>(y) + at) = make_uint4(h[0], h[1], h[2], h[3]);
+    // One 16-byte store, whose type asks for a half's alignment only (cx_exl3_output_transform's y).
+    typedef uint32_t HalfAligned4 __attribute__((ext_vector_type(4), aligned(2)));
+    *reinterpret_cast<HalfAligned4*>(static_cast<__half*>(y) + at) = HalfAligned4{h[0], h[1], h[2], h[3]};
   } else {
 #pragma unroll
     for (int i = 0; i < 8; ++i) v[i] *= sg * (kHadNorm * sv[i]);

@@ -86,7 +86,8 @@ int cx_exl3_input_transform(const cx_exl3_matrix* m, const void* x, int32_t x_dt
 /* The output transform alone: y = WHT128(y_raw) * (norm * svh) in fp32 (CX_F32, the
  * engine's LinOutBlock, engine/exl3/exl3.h:69-82) or fp16(RoundH(WHT128(RoundH(y_raw)) *
  * norm) * svh) (CX_F16, ref/exl3_ref.py:153-156, 175), per 128-block.  The parity hook for
- * the output transform cx_exl3_linear runs.  y_raw fp32 [M][out_features]; y [M][out_features]. */
+ * the output transform cx_exl3_linear runs.  y_raw fp32 [M][out_features]; y [M][out_features].
+ * y_raw and an fp32 y are 16-byte aligned; an fp16 y may start at any half. */
 int cx_exl3_output_transform(const cx_exl3_matrix* m, const float* y_raw, int32_t M, void* y, int32_t y_dtype,
                              cx_stream_t stream);
 

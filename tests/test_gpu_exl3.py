@@ -345,6 +345,24 @@ def test_output_transform_bit_exact(ops):
     _same_values(got, want)
 
 
+@pytest.mark.parametrize("shift", [1, 2, 3, 4])
+def test_output_transform_fp16_alignment(ops, shift):
+    # An fp16 y may start at any half: the same bits as at a 16-byte boundary, nothing beside them.
+    import ctypes
+    from exl3moe import check, lib
+    rng = np.random.default_rng(31)
+    M, O_ = 5, 256
+    lin = _plain_linear(ops, 128, O_, np.ones(128, np.float16), (rng.standard_normal(O_) + 0.1).astype(np.float16))
+    y = torch.from_numpy((rng.standard_normal((M, O_)) * 10).astype(np.float32)).cuda()
+    want = lin.output_transform(y, torch.float16)
+    buf = torch.full((M * O_ + 16,), 7.0, dtype=torch.float16, device="cuda")
+    check("cx_exl3_output_transform", lib().cx_exl3_output_transform(
+        ctypes.byref(lin.struct), y.data_ptr(), M, buf[shift:].data_ptr(), 0, None))
+    torch.cuda.synchronize()
+    assert torch.equal(buf[shift:shift + M * O_].view(torch.int16), want.flatten().view(torch.int16))
+    assert torch.all(buf[:shift] == 7.0) and torch.all(buf[shift + M * O_:] == 7.0)
+
+
 @pytest.mark.parametrize("seed", range(32))
 def test_random_linear(ops, seed):
     # Seeded random widths (128-2048 in 128 steps on either side), rate, codebook, row
