@@ -277,32 +277,6 @@ bool LaunchGemmTall(int k2, int cb, dim3 grid, const GemmArgs& g, hipStream_t s)
   }
 }
 
-// The many-row GEMM (Exl3GemmRowsKernel) or the few-row path for M rows of one matrix, by their
-// estimated times in us (whole calls at 4 bpw, 65-4,096 rows of 2048 -> 4096, 4096 -> 2048, 2048 -> 512
-// and 2048 -> 12288 measured: within ~15%).
-//   Few rows: ~13.5 + 9.6 ns per row and 1 M weights.
-//   Many rows: ~6 + per step (32 k) 0.21 + 0.05 per row block while at most 256 workgroups run (one
-//   per CU), 0.37 + 0.0625 per round of 512 (two per CU).
-// Measured, few / many rows: 2048 -> 4096 128 rows 21.6 / 22.9, 256 34 / 26, 2,048 182 / 62; 4096 -> 2048 256
-// rows 34 / 40, 512 54 / 44; 2048 -> 512 512 rows 17 / 23, 1,536 31 / 27.
-// nrb: the row blocks per entry of the cheapest many-row form; 0: the few-row path.
-int RowsBlocks(int M, int A, int ncp) {
-  if (M <= 64) return 0;
-  const int blocks = (M + 15) / 16, steps = A / 2;
-  double best = 13.5 + 0.0096e-6 * M * (16.0 * A) * (32.0 * ncp);
-  int nrb = 0;
-  for (int n = 1; n <= std::min(kRowsMaxBlocks, blocks); ++n) {
-    const long wgs = (long)((blocks + n - 1) / n) * (ncp / 4), rem = wgs % 512;
-    const double lone = 0.21 + 0.05 * n, full = 0.37 + 0.0625 * n;
-    const double us = 6.2 + steps * (wgs / 512 * full + (rem == 0 ? 0 : rem <= 256 ? lone : full));
-    if (us < best) {
-      best = us;
-      nrb = n;
-    }
-  }
-  return nrb;
-}
-
 size_t LinearWorkspace(const LinearPlan& p, int I, int O, int M) {
   return AlignUp((size_t)M * I * 2, 256) + AlignUp((size_t)p.S * M * O * 4, 256);
 }
@@ -351,11 +325,11 @@ int RunGroup(const cx_exl3_job* jobs, int n, int M, char* ws, hipStream_t s) {
   }
   hipLaunchKernelGGL(InputTransformKernel, dim3((unsigned)((in_items * 16 + 255) / 256)), dim3(256), 0, s, tin);
   // Many rows: transformed outputs straight from one GEMM, the jobs of one rate and codebook in
-  // one launch.  The group takes it when its largest job does.
-  const int big = (int)(std::max_element(gs.begin(), gs.end(),
-                                         [](const GemmArgs& a, const GemmArgs& b) { return a.A * a.ncp < b.A * b.ncp; }) -
-                        gs.begin());
-  if (RowsBlocks(M, gs[big].A, gs[big].ncp) > 0) {
+  // one launch, every job in entries of the same height.
+  RowsShape shapes[kMaxGroupJobs];
+  for (int j = 0; j < n; ++j) shapes[j] = RowsShape{gs[j].A, gs[j].ncp, ps[j].S, jobs[j].m.k2, jobs[j].m.codebook};
+  if (const int nrb = RowsBlocks(shapes, n, M)) {
+    const int entries = (M + 16 * nrb - 1) / (16 * nrb);
     std::vector<bool> done(n, false);
     for (int j = 0; j < n; ++j) {
       if (done[j]) continue;
@@ -363,8 +337,6 @@ int RunGroup(const cx_exl3_job* jobs, int n, int M, char* ws, hipStream_t s) {
       for (int i = j; i < n && gm.n < kMaxMultiJobs; ++i) {
         if (done[i] || jobs[i].m.k2 != jobs[j].m.k2 || jobs[i].m.codebook != jobs[j].m.codebook) continue;
         const GemmArgs& g = gs[i];
-        const int nrb = std::max(1, RowsBlocks(M, g.A, g.ncp));
-        const int entries = (M + 16 * nrb - 1) / (16 * nrb);
         gm.job[gm.n] = RowsJob{g.mat.tiles, g.mat.svh, g.plane[0].x, g.plane[0].y, jobs[i].y, jobs[i].ldy,
                                jobs[i].y_dtype == CX_F16 ? 1 : 0, M, g.A, g.ncp, ps[i].S, nrb, entries};
         gm.start[gm.n + 1] = gm.start[gm.n] + RowsJobGroups(entries, g.ncp);

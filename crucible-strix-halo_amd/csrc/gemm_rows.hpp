@@ -25,6 +25,7 @@
 #pragma once
 
 #include "gemm.hpp"
+#include "rows_rule.hpp"
 
 namespace cx {
 
@@ -171,8 +172,6 @@ __device__ __forceinline__ void RowsLoop(u32x4_t rw, u32x4_t rx, int ldx_bytes, 
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the last copies: the caller reuses their LDS
 }
 
-constexpr int kRowsMaxBlocks = 8;  // 16-row blocks of a workgroup
-
 struct RowsJob {
   const uint32_t* tiles;
   const __half* svh;
@@ -191,11 +190,6 @@ struct RowsMulti {
   int start[kMaxMultiJobs + 1];  // first workgroup of each job
   RowsJob job[kMaxMultiJobs];
 };
-// Workgroups of a job: entry e's column blocks on XCD e % 8 (ids go to the XCDs round-robin), so
-// its activation rows are fetched into one L2; with fewer than 16 entries in plain order.
-__host__ __device__ inline int RowsJobGroups(int entries, int ncp) {
-  return (entries < 16 ? entries : (entries + 7) / 8 * 8) * (ncp / 4);
-}
 
 template <int K2, int CB>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) Exl3GemmRowsKernel(RowsMulti gm) {

@@ -5,14 +5,14 @@ torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
 
 
-# Shapes that take the many-row GEMM: uneven K splits (60, 20 and 52 steps), 1 to 4 K segments
+# Shapes that take the many-row GEMM: uneven K splits (60, 20 and 52 steps), 1 to 8 K segments
 # (sums parked in the workspace), half-bit rates (weights copied every second chunk), entries in
 # plain and in XCD order, 1 to 8 row blocks per entry, last entries of every size.
 @pytest.mark.parametrize("I,Ot,bits,cb,rows", [
     (2048, 4096, 4, "mul1", (300, 2047)), (1920, 5120, 3, "mul1", (193, 1025)), (640, 12288, 2.5, "mul1", (129, 777)),
     (4096, 2048, 5, "mcg", (1290,)), (1664, 8192, 3.5, "mul1", (255,)), (8192, 1024, 6, "mul1", (2033,)),
     (1024, 16384, 8, "3inst", (65, 400)), (512, 24576, 1.5, "mul1", (96, 129)), (3072, 6144, 7, "mul1", (511,)),
-    (2048, 8192, 1, "3inst", (201,)), (2048, 8192, 2, "mul1", (1111,)),
+    (2048, 8192, 1, "3inst", (201,)), (2048, 8192, 2, "mul1", (1111,)), (256, 512, 3, "mul1", (81, 192)),
 ])
 def test_rows_linear_equals_few_row_path(I, Ot, bits, cb, rows):
     if not torch.cuda.is_available():
