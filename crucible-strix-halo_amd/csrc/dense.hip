@@ -4,10 +4,10 @@
 //   * up to 8 rows of fp32 x: one wave per output row, fp32 products and sums
 //     (DenseGemvKernel, engine/layers/ops.h:30-61);
 //   * more rows, or fp16 x: x rounded to fp16 (the reference packs it first,
-//     PrefillPackKernel) and v_mfma_f32_16x16x32_f16 with fp32 sums: up to 64 rows one
-//     workgroup per 16 outputs with K split over its 8 waves (DenseSplitKernel), above
-//     that tiles of 64 rows x 48-96 outputs through LDS (DenseTileKernel); rows that are not
-//     16-byte aligned, or widths that are no multiple of 64, take DenseMfmaKernel.
+//     PrefillPackKernel) and v_mfma_f32_16x16x32_f16 with fp32 sums: up to 64 rows and I a
+//     multiple of 256 one workgroup per 16 outputs with K split over its 8 waves
+//     (DenseSplitKernel); else, where I is a multiple of 64 and the rows are 16-byte aligned, tiles of
+//     64 rows x 48-96 outputs through LDS (DenseTileKernel); the rest takes DenseMfmaKernel.
 #include "internal.hpp"
 
 namespace cx {
@@ -149,7 +149,7 @@ __global__ void __launch_bounds__(256) DenseMfmaKernel(const __half* __restrict_
   }
 }
 
-// Many rows, 16-byte aligned: a 512-thread workgroup computes rows [64 bx, 64 bx + 64) x outputs
+// 16-byte aligned rows: a 512-thread workgroup computes rows [64 bx, 64 bx + 64) x outputs
 // [16 NB by, 16 NB (by + 1)).  Chunks of 64 k of its x rows and W rows are copied from memory straight
 // into LDS two chunks ahead, whole 128-byte lines; wave w multiplies row block w / 2 by all NB output
 // blocks over half w % 2 of the chunk's k, and the two halves' sums are added at the end.  Rows >= M
@@ -160,8 +160,8 @@ __global__ void __launch_bounds__(256) DenseMfmaKernel(const __half* __restrict_
 // weights that each workgroup reads again (186 MB in all) bound it.  Loading the MFMA fragments
 // from memory (16 bytes from each of 16 rows) gave ~35 bytes per ns and CU: 66 us a call with one
 // wave over all of K (DenseMfmaKernel), 31 us with K split over 8 waves; in whole lines into LDS
-// 15.5 us.  gridDim.x is a multiple of 8, so all workgroups of a row tile run on one XCD and its
-// x rows go into one L2 (3,000 rows: 35 -> 20 us).
+// 15.7 us.  gridDim.x is a multiple of 8 (but for few row tiles of many outputs), so all workgroups of a
+// row tile run on one XCD and its x rows go into one L2 (3,000 rows: 35 -> 20 us).
 template <bool XF32, int NB>
 __global__ void __launch_bounds__(512) DenseTileKernel(const __half* __restrict__ W, int O, int I,
                                                        const void* __restrict__ x, int ldx, int M, float* __restrict__ y,
@@ -433,10 +433,15 @@ int cx_dense_linear(const uint16_t* W, int32_t O, int32_t I, const void* x, int3
         nb = n;
       }
     }
+    // Row tiles in the grid: whole groups of 8, so that each tile's workgroups share one XCD's L2.  Fewer
+    // than 8 tiles then leave the other XCDs idle, which costs nothing while a tile's workgroups fit the
+    // XCD's 32 CUs; above that they are spread over all XCDs.  Shared / spread: 65 rows, 513 outputs over
+    // 2,048 fp16 9.8 / 10.3 us; 2,049 outputs over 1,920 fp32 19.3 / 12.8.
+    const int gx = mt < 8 && (ob + nb - 1) / nb > 32 ? mt : (mt + 7) / 8 * 8;
     auto go = [&](auto f32c, auto nbc) {
       constexpr bool F32 = decltype(f32c)::value != 0;
       constexpr int NB = decltype(nbc)::value;
-      hipLaunchKernelGGL((DenseTileKernel<F32, NB>), dim3((mt + 7) / 8 * 8, (ob + NB - 1) / NB), dim3(512), 0, s, w, O, I, x, ldx, M, y, ldy);
+      hipLaunchKernelGGL((DenseTileKernel<F32, NB>), dim3(gx, (ob + NB - 1) / NB), dim3(512), 0, s, w, O, I, x, ldx, M, y, ldy);
     };
     auto width = [&](auto f32c) {
       switch (nb) {

@@ -6,11 +6,13 @@ torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
 
 
-# One chunk of 64 k, odd chunk counts, 48- to 96-output tiles with 1-output remainders, row tiles of
-# 1 to 64 rows in grids that are no multiple of 8, padded and unaligned rows.
+# One chunk of 64 k, odd chunk counts, 48-output tiles with remainders, row tiles of 1 to 64 rows in
+# grids that are no multiple of 8, padded and unaligned rows; fewer than 8 row tiles of many outputs
+# (spread over the XCDs).
 @pytest.mark.parametrize("M,I,Ot,pad", [
     (65, 64, 1, 0), (127, 128, 49, 0), (192, 192, 65, 8), (577, 320, 97, 0), (300, 2048, 513, 0), (1100, 2048, 257, 24),
     (70, 96, 33, 0), (201, 160, 100, 0), (130, 64, 70, 1), (99, 256, 17, 3), (2113, 64, 81, 0),
+    (65, 128, 1585, 0), (384, 192, 2049, 8), (17, 64, 1600, 0),
 ])
 @pytest.mark.parametrize("dt", ["float32", "float16"])
 def test_dense_tiles(M, I, Ot, pad, dt):
