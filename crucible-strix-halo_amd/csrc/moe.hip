@@ -726,7 +726,7 @@ __global__ void __launch_bounds__(256) MoeCombineKernel(const void* __restrict__
 // and kept in it, so each plan runs one fixed configuration:
 //   CX_PREFILL_NRB (4 | 8) and CX_PREFILL_WPG (4 | 8 | 16): a register-blocked prefill
 //     workgroup of wpg waves covers 16 nrb rows x 32 wpg columns;
-//   CX_PREFILL_GEMM: 0 register-blocked, 1 tall, -1 by the rows per expert;
+//   CX_PREFILL_GEMM: 0 register-blocked, 1 tall, -1 by the rows per expert and the workgroups;
 //   CX_PREFILL_MID: the mid fused into the register-blocked gate/up GEMM (needs nrb = 4);
 //   CX_TALL_SEQMID: tall prefill with gate, up and the mid in one workgroup, one plane after
 //     the other (0: separate plane workgroups and a mid launch);
@@ -796,8 +796,18 @@ MoeSizes PlanMoe(const cx_moe_plan* pl, int M, int mode) {
   s.nrb = decode ? 1 : ps.nrb;
   s.wpg = decode ? 4 : ps.wpg;
   // The tall GEMM when experts average at least 96 rows (one decode then serves up to 192
-  // rows); below that most entries fit the register-blocked GEMM's 64 rows.
-  const int kern = ps.kernel >= 0 ? ps.kernel : (long)M * pl->topk >= 96L * pl->E ? 1 : 0;
+  // rows); below that most entries fit the register-blocked GEMM's 64 rows.  Register-blocked / tall,
+  // layers of 512 experts, top-10, H = 2048, I = 512 at 4 bpw, evenly routed: 64 rows an expert 670 / 677 us,
+  // 96 954 / 845, 160 1,461 / 1,261; routed by Zipf weights 80 833 / 841, 96 967 / 959, 160 1.06x.
+  //
+  // Not where its gate/up workgroups (192 rows x 128 columns) are fewer than half the CUs, for codebooks
+  // whose decode costs more than mul1's: the launch then takes as long as one workgroup, and that is longer
+  // than before the tall form copied whole rows (8 experts, top-2, H = 1024, I = 512, 8 bpw mcg, 1,200 rows:
+  // before / tall / register-blocked 106.9 / 111.7 / 75.4 us; 4 bpw mul1 105.2 / 100.6 / 64.9).
+  const long expert_rows = (long)M * pl->topk / pl->E, tall_rows = 64 * kTallRowBlocksPerWave;
+  const long tall_groups = (pl->E * ((expert_rows + tall_rows - 1) / tall_rows) + (M + tall_rows - 1) / tall_rows) * (pl->I / 128);
+  const bool tall_idle = pl->cb_gu != kCbMul1 && ps.nrb == 4 && ps.mid && tall_groups < 128;
+  const int kern = ps.kernel >= 0 ? ps.kernel : (long)M * pl->topk >= 96L * pl->E && !tall_idle ? 1 : 0;
   s.tall = !decode && kern == 1;
   if (s.tall) s.nrb = 4 * kTallRowBlocksPerWave;
   // Register-blocked prefill: gate and up in one workgroup with the mid fused into the
@@ -853,7 +863,9 @@ MoeSizes PlanMoe(const cx_moe_plan* pl, int M, int mode) {
   s.off_xg = take((size_t)s.P * pl->H * 2);
   s.off_xu = take((size_t)s.P * pl->H * 2);
   s.off_yg = take((size_t)s.P * pl->I * 4);
-  s.off_yu = take((size_t)s.P * pl->I * 4);
+  // The fused mid needs neither raw plane; where it stands in for the tall form the workspace is
+  // no larger than that form's (its entry table is shorter).
+  s.off_yu = s.mid && tall_idle ? s.off_yg : take((size_t)s.P * pl->I * 4);
   s.off_xd = take((size_t)s.P * pl->I * 2);
   s.off_yd = take((size_t)s.P * pl->H * (s.prefill ? 2 : 4));
   s.off_ysc = take(s.prefill ? (size_t)s.P * (pl->H / 128) * 4 : 0);

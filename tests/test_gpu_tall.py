@@ -43,3 +43,24 @@ def test_tall_entries(monkeypatch, H, Ie, bgu, bd, cb, seq):
         y = tall.cpu().numpy()
         assert rel_l2(y, ref) <= 1e-3  # the layer tests' bounds
         assert np.abs(y - ref).max() <= 2e-3 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("cb,idle", [("mcg", True), ("3inst", True), ("mul1", False)])
+def test_tall_not_on_an_idle_chip(monkeypatch, cb, idle):
+    # 8 experts of more than 96 rows, I = 256: 22 gate/up workgroups of the tall form.  In the mcg and 3inst
+    # codebooks the register-blocked form runs, in a workspace no larger than the tall form's.
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from exl3moe import CX_MOE_PREFILL, synth
+    monkeypatch.delenv("CX_PREFILL_GEMM", raising=False)
+    make = lambda: synth.device_moe_layer(9, E=8, H=256, Ie=256, topk=2, codebook=cb)
+    plan = make()
+    monkeypatch.setenv("CX_PREFILL_GEMM", "1")
+    tall = make()
+    M = 500
+    assert (plan.workspace_size(M, CX_MOE_PREFILL) < tall.workspace_size(M, CX_MOE_PREFILL)) == idle
+    g = torch.Generator(device="cuda").manual_seed(1)
+    x = torch.randn(M, 256, device="cuda", generator=g).half()
+    lg = torch.randn(M, 9, device="cuda", generator=g)
+    a, b = plan(x, lg, mode=CX_MOE_PREFILL), tall(x, lg, mode=CX_MOE_PREFILL)
+    assert torch.equal(a.view(torch.int32), b.view(torch.int32))
