@@ -371,22 +371,47 @@ __device__ __forceinline__ void StorePerm32x8LdsBuf(uint32_t* area, __amdgpu_buf
 
 // Asynchronous copies from a buffer into LDS (no registers): lane l's N consecutive dwords (N = 1
 // or 4; the 3-dword form does not pack its lanes) at byte offset voff + soff land at lds + 4 N l
-// (offsets past the buffer give zeros).
+// (offsets past the buffer give zeros).  C copies: copy i at soff + i sstep, to lds + i LSTEP.
 // Written as assembly, so that the compiler's own waits neither count these copies nor hold
 // LDS reads back for them: the caller waits with WaitLoadsBarrier before the reads, and drains
 // the copies before the LDS is used for something else.
 // The compiler puts no wait states into assembly: s_mov and s_nop 3 are the five that lie between a
-// VALU write of a scalar operand (v_readfirstlane, a spilled SGPR's v_readlane) and the load reading
-// it, and the one between the write of m0 and its use.
+// VALU write of a scalar operand (v_readfirstlane, a spilled SGPR's v_readlane) and the first load
+// reading it; inside the run only scalar instructions write, which need none, but for the one between
+// m0's write and its use.  One statement for the run, so that nothing comes in between: with a statement
+// and the wait states for each copy the router product of 65 rows took 13.0 us instead of 12.3, of 2,048
+// rows 16.1 instead of 15.6.
 typedef __attribute__((address_space(3))) char LdsChar;
-template <int N>
-__device__ __forceinline__ void CopyToLds(u32x4_t rsrc, uint32_t voff, uint32_t soff, uint32_t lds) {
-  static_assert(N == 1 || N == 4, "a copy moves 1 or 4 dwords per lane");
-  if constexpr (N == 1)
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "memory", "m0");
-  else
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "memory", "m0");
+#define CX_COPY_FIRST(W) "s_mov_b32 m0, %3\n\ts_nop 3\n\tbuffer_load_dword" W " %1, %2, %0 offen lds"
+#define CX_COPY_NEXT(W) "\n\ts_add_u32 m0, m0, %5\n\ts_add_u32 %0, %0, %4\n\tbuffer_load_dword" W " %1, %2, %0 offen lds"
+#define CX_COPY_RUN(C, TEXT)                                                                                        \
+  case C:                                                                                                           \
+    asm volatile(TEXT : "+&s"(soff) : "v"(voff), "s"(rsrc), "s"(lds), "s"(sstep), "n"(LSTEP) : "memory", "m0", "scc"); \
+    break
+template <int N, int C = 1, int LSTEP = 0>
+__device__ __forceinline__ void CopyToLds(u32x4_t rsrc, uint32_t voff, uint32_t soff, uint32_t lds, uint32_t sstep = 0) {
+  static_assert((N == 1 || N == 4) && C >= 0 && C <= 6, "up to 6 copies of 1 or 4 dwords per lane");
+  if constexpr (N == 1) {
+    switch (C) {
+      CX_COPY_RUN(1, CX_COPY_FIRST(""));
+      CX_COPY_RUN(2, CX_COPY_FIRST("") CX_COPY_NEXT(""));
+      CX_COPY_RUN(3, CX_COPY_FIRST("") CX_COPY_NEXT("") CX_COPY_NEXT(""));
+      default: static_assert(N != 1 || C <= 3, "not written");
+    }
+  } else {
+    switch (C) {
+      CX_COPY_RUN(1, CX_COPY_FIRST("x4"));
+      CX_COPY_RUN(2, CX_COPY_FIRST("x4") CX_COPY_NEXT("x4"));
+      CX_COPY_RUN(3, CX_COPY_FIRST("x4") CX_COPY_NEXT("x4") CX_COPY_NEXT("x4"));
+      CX_COPY_RUN(4, CX_COPY_FIRST("x4") CX_COPY_NEXT("x4") CX_COPY_NEXT("x4") CX_COPY_NEXT("x4"));
+      CX_COPY_RUN(5, CX_COPY_FIRST("x4") CX_COPY_NEXT("x4") CX_COPY_NEXT("x4") CX_COPY_NEXT("x4") CX_COPY_NEXT("x4"));
+      CX_COPY_RUN(6, CX_COPY_FIRST("x4") CX_COPY_NEXT("x4") CX_COPY_NEXT("x4") CX_COPY_NEXT("x4") CX_COPY_NEXT("x4") CX_COPY_NEXT("x4"));
+    }
+  }
 }
+#undef CX_COPY_RUN
+#undef CX_COPY_NEXT
+#undef CX_COPY_FIRST
 // Raw buffer words for CopyToLds (as MakeRsrc).
 __device__ __forceinline__ u32x4_t MakeRsrcWords(const void* base, uint32_t bytes) {
   const uint64_t a = reinterpret_cast<uint64_t>(base);

@@ -183,20 +183,19 @@ __global__ void __launch_bounds__(512) DenseTileKernel(const __half* __restrict_
   // Piece p of row r lies in slot p ^ (r & 7): the 8 rows of a fragment read cover all banks.
   const int xr = lane / XP, wr = lane >> 3;
   const uint32_t lds = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)(LdsChar*)smem);
+  // Wave w does the copies t = w, w + 8, ...: first CX of x (voff: its rows are those of t = w, 8 on from copy
+  // to copy), then of W; (XI + WI) % 8 waves have one more of W.
+  constexpr int CX = XI / 8, CW = NC - CX, XR = 1024 / XB;
+  const int xrow = wave * XR + xr;
+  const uint32_t xv = (uint32_t)(xr * ldx * esz + 16 * ((lane % XP) ^ (xrow & 7))), wv = (uint32_t)(wr * I * 2 + 16 * ((lane & 7) ^ wr));
   auto copy = [&](int c, int buf) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i <= NC; ++i) {
-      const int t = 8 * i + wave;
-      if (i == NC && wave >= NX) break;  // wave-uniform
-      const uint32_t dst = lds + buf * CB + t * 1024;
-      if (t < XI) {
-        const int r = t * (1024 / XB) + xr;
-        CopyToLds<4>(rx, (uint32_t)(xr * ldx * esz + 16 * ((lane % XP) ^ (r & 7))),
-                     (uint32_t)(t * (1024 / XB) * ldx * esz + c * XB), dst);
-      } else {
-        CopyToLds<4>(rw, (uint32_t)(wr * I * 2 + 16 * ((lane & 7) ^ wr)), (uint32_t)((t - XI) * 8 * I * 2 + c * 128), dst);
-      }
-    }
+    const uint32_t dst = lds + buf * CB + wave * 1024;
+    CopyToLds<4, CX, 8192>(rx, xv, (uint32_t)(wave * XR * ldx * esz + c * XB), dst, (uint32_t)(8 * XR * ldx * esz));
+    const uint32_t ws = (uint32_t)(wave * 8 * I * 2 + c * 128), wd = dst + CX * 8192;
+    if (wave < NX)  // wave-uniform
+      CopyToLds<4, CW + 1, 8192>(rw, wv, ws, wd, (uint32_t)(64 * I * 2));
+    else if constexpr (CW > 0)
+      CopyToLds<4, CW, 8192>(rw, wv, ws, wd, (uint32_t)(64 * I * 2));
   };
   const int rb = wave >> 1, kh = wave & 1, ln = lane & 15, q = lane >> 4;
   const int ar = 16 * rb + ln;

@@ -68,9 +68,7 @@ __device__ __forceinline__ void RowsLoop(u32x4_t rw, u32x4_t rx, int ldx_bytes, 
   constexpr int XL = (NA + 1) / 2;
   const uint32_t xoff = (uint32_t)((wave * 8 + (lane >> 3)) * ldx + 16 * ((lane & 7) ^ (lane >> 3)));
   auto load_x = [&](int c, int buf) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < XL; ++i)
-      CopyToLds<4>(rx, xoff, (uint32_t)(c * 128 + i * 32 * ldx), xlds + buf * CBYTES + (4 * i + wave) * 1024);
+    CopyToLds<4, XL, 4096>(rx, xoff, (uint32_t)(c * 128), xlds + buf * CBYTES + wave * 1024, 32u * (uint32_t)ldx);
   };
   uint32_t xrd[2];  // the lane's fragment of the chunk's step j, row block 0
 #pragma unroll
@@ -82,11 +80,8 @@ __device__ __forceinline__ void RowsLoop(u32x4_t rw, u32x4_t rx, int ldx_bytes, 
   constexpr int NW = WD / 4 + WD % 4;       // its instructions: 4 dwords per lane, then single ones
   auto load_w = [&](int c, int buf) __attribute__((always_inline)) {  // PAIRED: c and buf even
     const uint32_t so = (uint32_t)(c * WBYTES), l = wlds + buf * WBYTES;
-#pragma unroll
-    for (int k = 0; k < WD / 4; ++k) CopyToLds<4>(rw, (uint32_t)lane * 16, so + 1024 * k, l + 1024 * k);
-#pragma unroll
-    for (int k = 0; k < WD % 4; ++k)
-      CopyToLds<1>(rw, (uint32_t)lane * 4, so + 1024 * (WD / 4) + 256 * k, l + 1024 * (WD / 4) + 256 * k);
+    if constexpr (WD / 4 > 0) CopyToLds<4, WD / 4, 1024>(rw, (uint32_t)lane * 16, so, l, 1024u);
+    if constexpr (WD % 4 > 0) CopyToLds<1, WD % 4, 256>(rw, (uint32_t)lane * 4, so + 1024 * (WD / 4), l + 1024 * (WD / 4), 256u);
   };
   auto read_windows = [&](uint32_t (&v)[2][3], int buf, int j) __attribute__((always_inline)) {
 #pragma unroll

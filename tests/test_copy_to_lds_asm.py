@@ -26,6 +26,15 @@ extern "C" __global__ void OffsetFromLane(const uint32_t* src, uint32_t* out, in
   WaitLoadsBarrier<0>();
   out[threadIdx.x] = s[threadIdx.x];
 }
+// Runs of copies.
+extern "C" __global__ void Runs(const uint32_t* src, uint32_t* out, int n) {
+  __shared__ __align__(16) uint32_t s[2048];
+  const uint32_t lds = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)(LdsChar*)s);
+  CopyToLds<4, 6, 1024>(MakeRsrcWords(src, 65536), threadIdx.x * 16, 64, lds, (uint32_t)n);
+  CopyToLds<1, 3, 256>(MakeRsrcWords(src, 65536), threadIdx.x * 4, 64, lds + 6144, 256u);
+  WaitLoadsBarrier<0>();
+  out[threadIdx.x] = s[threadIdx.x];
+}
 // m0 holds the same value for another instruction before and after the copy (compiled, never run).
 extern "C" __global__ void OtherUseOfM0(const uint32_t* src, uint32_t* out, int a) {
   __shared__ __align__(16) uint32_t s[1024];
@@ -46,7 +55,7 @@ def kernels(tmp_path_factory):
     src.write_text(f'#include "{CSRC}/common.hpp"\n{SRC}')
     text = subprocess.run([HIPCC, *FLAGS, "-S", str(src), "-o", "-"], check=True, capture_output=True, text=True).stdout
     out = {}
-    for name in ("OffsetFromLane", "OtherUseOfM0"):
+    for name in ("OffsetFromLane", "Runs", "OtherUseOfM0"):
         body = re.search(rf"^{name}:.*?s_endpgm", text, re.S | re.M).group(0)
         out[name] = [ln.split(";")[0].strip() for ln in body.splitlines() if re.match(r"\s+[sv]_|\s+(buffer|global|ds)_", ln)]
     return out
@@ -75,6 +84,21 @@ def test_wait_states_before_the_load(kernels):
             m = re.match(r"s_nop (\d+)", c)
             states += int(m.group(1)) + 1 if m else 1
     assert seen >= 2  # both forms were compiled with an offset from a VALU write
+
+
+def test_runs_advance_offset_and_m0(kernels):
+    # Each further copy: m0 and the offset advanced by scalar instructions, one of them between m0's write
+    # and the load (m0's wait state); nothing else between the copies of a run.
+    code = kernels["Runs"]
+    loads = [i for i, c in enumerate(code) if re.match(r"buffer_load.* lds$", c)]
+    assert [c.split()[0] for c in code if re.match(r"buffer_load.* lds$", c)] == 6 * ["buffer_load_dwordx4"] + 3 * ["buffer_load_dword"]
+    for i, j in zip(loads, loads[1:]):
+        if i == loads[5]:
+            continue  # from the first run to the second
+        off = re.search(r", (s\d+) offen", code[j]).group(1)
+        assert j == i + 3
+        assert re.match(r"s_add_u32 m0, m0, 0x(400|100)$", code[i + 1]), code[i:j + 1]
+        assert re.match(rf"s_add_u32 {off}, {off}, s\d+$", code[i + 2]), code[i:j + 1]
 
 
 def test_m0_is_set_again_after_a_copy(kernels):
