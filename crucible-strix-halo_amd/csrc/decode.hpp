@@ -93,7 +93,8 @@ __device__ __forceinline__ uint32_t CodeTerm(uint32_t r) {
 // rounding, docs/EXL3_FORMAT.md:120-131) on the pair.  v_sad_u8 and not v_dot4_u32_u8: both
 // issue in ~4.3 cycles, but a dot product runs on the matrix pipe and hides nothing behind an
 // MFMA (64 of them with 16 MFMAs, 2 waves per SIMD: 560 cycles, 64 v_sad_u8 461).  Config-size
-// layer calls: 2,048 rows 490 -> 483 us, 8,192 rows 1,296 -> 1,273, 61 rows 179 -> 177.
+// layer calls: 2,048 rows 490 -> 483 us, 8,192 rows 1,296 -> 1,273; decode calls within 1%, no more
+// than two runs of one build differ.
 template <int CB>
 __device__ __forceinline__ half2_t PairWeights(uint32_t a, uint32_t b) {
   if constexpr (CB == kCbMul1) {

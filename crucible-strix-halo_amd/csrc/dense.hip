@@ -160,7 +160,7 @@ __global__ void __launch_bounds__(256) DenseMfmaKernel(const __half* __restrict_
 // weights that each workgroup reads again (186 MB in all) bound it.  Loading the MFMA fragments
 // from memory (16 bytes from each of 16 rows) gave ~35 bytes per ns and CU: 66 us a call with one
 // wave over all of K (DenseMfmaKernel), 31 us with K split over 8 waves; in whole lines into LDS
-// 15.7 us.  gridDim.x is a multiple of 8 (but for few row tiles of many outputs), so all workgroups of a
+// 15.9 us (kernel times).  gridDim.x is a multiple of 8 (but for few row tiles of many outputs), so all workgroups of a
 // row tile run on one XCD and its x rows go into one L2 (3,000 rows: 35 -> 20 us).
 template <bool XF32, int NB>
 __global__ void __launch_bounds__(512) DenseTileKernel(const __half* __restrict__ W, int O, int I,

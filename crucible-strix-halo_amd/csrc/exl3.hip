@@ -13,10 +13,11 @@ namespace cx {
 // dwords of a tile are its 16K little-endian int16 words unchanged, so a column pair's two
 // tiles are 2 T dwords in one piece on both sides, U units of type V: a transpose of pieces.
 //
-// Bound by HBM.  A thread moves one unit of four consecutive a's: 16-byte accesses, one
+// Bound by memory.  A thread moves one unit of four consecutive a's: 16-byte accesses, one
 // division per four, and each pair's four pieces (128 k2 bytes) are whole lines at every rate.
-// 2048 x 32768 at 4 bpw (67 MB moved): 20 us by dwords with two 64-bit divisions each,
-// 11 so.
+// 2048 x 32768 at 4 bpw (67 MB moved), repeated on the same tensors, which then lie partly in the
+// Infinity Cache: 20 us by dwords with two 64-bit divisions each, 11 so.  A first call on new
+// tensors, its host part included: 44 and 37 us.
 template <class V>
 __global__ void __launch_bounds__(256) RepackKernel(const V* __restrict__ src, V* __restrict__ dst, int A, int ncp,
                                                     uint32_t U) {

@@ -932,7 +932,8 @@ namespace cx {
 // Bound by the decode's issue (289 cycles of a SIMD per wave-step, two column runs) with the MFMAs
 // beside it, which hide about half of their 17 cycles each.  Against 32-k activation tiles (64-byte
 // pieces of rows, a barrier per step, three waves per SIMD), gate/up with the mid: 2,048 Zipf-routed
-// rows at 4 bpw 271 -> 253 us, 199 rows 189 -> 166, 600 rows 209 -> 183, 2,048 rows at 8 bpw 364 -> 296.
+// rows at 4 bpw 271 -> 253 us, 199 rows 189 -> 166, 600 rows 209 -> 183, 2,048 rows at 8 bpw 364 -> 296
+// (both sides in short runs; calls repeated until the clocks settle: 250 us at 2,048 rows, 153 at 199).
 template <int K2, int CB>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) Exl3GemmPrefillMidKernel(GemmArgs g) {
   constexpr int NRB = 4, WPP = 4;  // row blocks of an entry, waves (column pairs) per plane

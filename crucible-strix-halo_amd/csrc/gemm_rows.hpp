@@ -12,11 +12,12 @@
 //
 // Bound by issue: a step of a wave (32 k x 32 columns) is 62 VALU of decode (289 cycles at 4
 // bpw) and 2 NRB MFMAs of 17 cycles, which leave the VALU about half of their time: ~440 cycles
-// for 8 row blocks.  2048 -> 4096 at 4 bpw, 2,048 rows: 56 us (616 TFLOP/s), without its epilogue
-// 50, its sums 45, its decode 41, its MFMAs 35; the few-row path's GEMM took 158 us and its output
-// transform 15.  With the activations and weights staged through registers instead the loop ran
-// as long (56.7 us) but spilled at 7 and 8 bpw and in the mcg and 3inst codebooks; reading the
-// windows a step earlier gained nothing (60 us).
+// for 8 row blocks.  2048 -> 4096 at 4 bpw, 2,047 rows: 52 us (657 TFLOP/s) with settled clocks.  Parts
+// taken out, in shorter runs where the whole took 56: without its epilogue 50, its sums 45, its
+// decode 41, its MFMAs 35; the few-row path's GEMM took 158 us there and its output transform 15.
+// With the activations and weights staged through registers instead the loop ran as long (56.7 us)
+// but spilled at 7 and 8 bpw and in the mcg and 3inst codebooks; reading the windows a step earlier
+// gained nothing (60 us).
 //
 // Sums: K in the few-row path's splits (4 S of them, LinearPlan), added in its order, so a
 // row's result is bitwise the same in either path.  Three levels: the split's MFMA
@@ -314,7 +315,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) E
 // then runs the up plane over the same entry and columns and computes the mid in the epilogue
 // (grid z = 1).
 //
-// 8,192 rows of 160 an expert, 3 / 5 bpw: gate/up with the mid 640 -> 566 us, down 397 -> 392, against
+// 8,192 rows of 160 an expert, 3 / 5 bpw, settled clocks: gate/up with the mid 640 -> 547-566 us, down
+// 397 -> 380-392 (the first launches after a pause, clocks unsettled: ~640 and ~450), against
 // a form that passed the decoded fragments between the waves through LDS and loaded activation
 // fragments straight from memory (16 bytes from each of 16 rows per load).  A gate/up workgroup's
 // two loops take 88 us (0.69 us a step of two waves per SIMD: ~0.45 is the MFMAs' and the decode's

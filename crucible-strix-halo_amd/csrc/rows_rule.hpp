@@ -24,8 +24,8 @@ constexpr int RowsJobGroups(int entries, int ncp) { return (entries < 16 ? entri
 //   Few rows: waves of A / (8 S) steps (32 k) for each 64 rows, 256 workgroups a round.
 //   Many rows: a step of a wave decodes one column pair (p below: by rate and codebook) and multiplies n row
 //   blocks; up to 256 workgroups run one per CU, further ones two per CU, 512 a round.
-// Fitted to 4,356 calls in both forms (1-8 bpw, three codebooks, 18 shapes and groups, 65-4,096 rows): 95% of
-// the few-row times within 11%, of the many-row ones within 8%.  The chosen form is on average 0.3%
+// Fitted to 4,356 calls in both forms (1-8 bpw, three codebooks, 18 shapes and groups, 65-4,096 rows): 97% of
+// the few-row times are met within 15%, 94% of the many-row ones within 10%.  The chosen form is on average 0.3%
 // above the best of all nine; 11 of the calls are more than 3%, none more than 6.1% above the few-row path.
 // Few rows / many rows measured: 2048 -> 4096 128 rows 22.7 / 24.7 (3inst 8 bpw 23.4 / 36.6), 512 rows
 // 56.5 / 33.9 (57 / 46), 2,048 rows 181 / 64; 2048 -> 512 1,024 rows 26.3 / 26.9 (26.5 / 39.3).
